@@ -408,7 +408,7 @@ def time_linear(dev, k, n, bits, rows_list, steps=20):
             for i in order:
                 mods[i].forward(x, {}, out_dtype=torch.float16)
         us = replay_median(graph, steps)[0]
-        path = ("gemv" if rows <= V.AUTO_RECONSTRUCT_THRESHOLD else
+        path = ("gemv" if rows <= V.AUTO_RECONSTRUCT_THRESHOLD else "gemm" if rows <= V.GEMM_MAX_ROWS else
                 "reconstruct_folded" if rows >= V.FUSED_RECONSTRUCT_MIN_ROWS else "reconstruct")
         res[str(rows)] = {"us": round(us, 2), "path": path,
                           "tflops": round(2.0 * rows * k * n / (us * 1e-6) / 1e12, 1)}

@@ -49,6 +49,27 @@ static int dequant_impl(const int16_t* trellis, int64_t k, int64_t n, int bits, 
     return 0;
 }
 
+// Rows [0, R), R <= GEMM_MAX_ROWS, by the GEMM kernels.
+static int gemm_slab(const uint16_t* a, int R, int64_t k, const int16_t* b, int64_t n, int bits, int codebook,
+                     const uint16_t* suh, const uint16_t* svh, void* c, int c_kind, void* scratch, int cus,
+                     hipStream_t s) {
+    const GemmPlan g = gemm_plan(R, k, n, cus);
+    u32x4_t* xd = reinterpret_cast<u32x4_t*>(scratch);
+    float4_t* partials = reinterpret_cast<float4_t*>(reinterpret_cast<char*>(scratch) + align_up(g.xd_bytes, 256));
+    const bool xcd = xcd_order_allowed() && g.n_hb % N_XCD == 0;
+    const int64_t waves = (int64_t)(R + 3) / 4 * (k / 128);
+    hipLaunchKernelGGL(gemm_rotate_kernel<0>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, a, suh, R, (int)k,
+                       g.n_rt * 16 * g.rb, xd);
+    int rc = check_launch();
+    if (rc) return rc;
+    const GemmArgs args{xd, b, (int)k, (int)n, g, codebook, partials, xcd, s};
+    EXL3_BITS_SWITCH(bits, rc = launch_gemm<B_>(args));
+    if (rc) return rc;
+    hipLaunchKernelGGL(gemm_finish_kernel<0>, dim3((unsigned)(g.n_hb * ((R + 15) / 16))), dim3(2 * WAVE), 0, s,
+                       partials, svh, c, c_kind, R, (int)n, g.n_kc, g.n_rt * g.rb, xcd ? 1 : 0);
+    return check_launch();
+}
+
 extern "C" {
 
 int exl3_dequant(const int16_t* trellis, int64_t k, int64_t n, int bits, int codebook,
@@ -82,7 +103,11 @@ int exl3_had_rows(const void* x, int x_kind, void* y, int y_kind, int64_t rows, 
 int64_t exl3_gemm_scratch_bytes(int64_t m, int64_t k, int64_t n) {
     clear_error();
     if (m <= 0 || k <= 0 || n <= 0) return fail("dimensions must be positive");
-    return gemv_scratch_bytes(m, k, n, device_cus());
+    // enough for every call of up to m rows: a k-chunk count may fall as the rows grow
+    const int cus = device_cus();
+    int64_t most = 0;
+    for (int64_t r = 1; r <= m && r <= GEMM_MAX_ROWS; ++r) most = std::max(most, dense_scratch_bytes(r, k, n, cus));
+    return most;
 }
 
 int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t n, int bits,
@@ -96,25 +121,28 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
     if (n <= 0 || n % 128) return fail("n must be a positive multiple of 128");
     if (c_kind < OUT_F16 || c_kind > OUT_F32) return fail("c_kind must be 0 (fp16), 1 (bf16) or 2 (fp32)");
     const int cus = device_cus();
-    if (scratch_bytes < gemv_scratch_bytes(m, k, n, cus)) return fail("scratch too small");
+    if (scratch_bytes < dense_scratch_bytes(m, k, n, cus)) return fail("scratch too small");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const GemvPlan p = gemv_plan(m, k, n, cus);
-    int* counters = reinterpret_cast<int*>(scratch);
-    float* partials = reinterpret_cast<float*>(reinterpret_cast<char*>(scratch) +
-                                               align_up((int64_t)p.n_cb * 4, 256));
     const size_t c_elem = c_kind == OUT_F32 ? 4 : 2;
-    const int64_t block = gemv_block_rows(m);
-    for (int64_t r0 = 0; r0 < m; r0 += block) {
-        const int R = (int)(m - r0 < block ? m - r0 : block);
+    const bool gemm = gemm_takes(m, k, n);
+    const int64_t slab = gemm ? GEMM_MAX_ROWS : GEMV_MAX_ROWS;
+    for (int64_t r0 = 0; r0 < m; r0 += slab) {
+        const int R = (int)std::min(m - r0, slab);
         const uint16_t* ar = a + r0 * k;
         void* cr = reinterpret_cast<char*>(c) + (size_t)r0 * n * c_elem;
-        const GemvArgs args{ar, b, suh, svh, cr, c_kind, R, (int)k, (int)n, p, codebook, counters, partials, s};
         int rc = 0;
+        if (gemm_takes(R, k, n)) {
+            if ((rc = gemm_slab(ar, R, k, b, n, bits, codebook, suh, svh, cr, c_kind, scratch, cus, s))) return rc;
+            continue;
+        }
+        const GemvPlan p = gemv_plan(R, k, n, cus);
+        float* partials = reinterpret_cast<float*>(scratch);
+        const GemvArgs args{ar, b, suh, svh, cr, c_kind, R, (int)k, (int)n, p, codebook, partials, s};
         EXL3_BITS_SWITCH(bits, rc = launch_gemv<B_>(args));
         if (rc) return rc;
-        if (p.split_reduce) {
-            hipLaunchKernelGGL(gemv_reduce_kernel<RED_BATCH>, dim3((int)(n / 128) * R), dim3(64), 0, s, partials, svh, cr,
-                               c_kind, R, (int)n, p.n_kc, p.xcd ? 1 : 0);
+        if (p.n_kc > 1) {
+            hipLaunchKernelGGL(gemv_reduce_kernel<RED_BATCH>, dim3((unsigned)(p.n_hb * R)), dim3(64), 0, s, partials,
+                               svh, cr, c_kind, R, (int)n, p.n_kc, p.xcd ? 1 : 0);
             if ((rc = check_launch())) return rc;
         }
     }
@@ -125,14 +153,15 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
 // member's region 256-byte aligned.
 static int64_t fan_scratch(int64_t m, int64_t k, int64_t count, const int64_t* n_list, int cus, GemvPlan* plan,
                            int64_t* offsets) {
-    int64_t total_cb = 0;
-    for (int64_t j = 0; j < count; ++j) total_cb += (n_list[j] + COLS - 1) / COLS;
-    const GemvPlan p = gemv_fan_plan(m, k, total_cb, cus);
+    int64_t total_hb = 0;
+    for (int64_t j = 0; j < count; ++j) total_hb += n_list[j] / GEMV_COLS;
+    GemvPlan p = gemv_plan_hb(m, k, total_hb, cus);
+    p.xcd = xcd_order_allowed() && total_hb % N_XCD == 0;
     const int64_t rows = m < GEMV_MAX_ROWS ? m : GEMV_MAX_ROWS;
     int64_t o = 0;
     for (int64_t j = 0; j < count; ++j) {
         if (offsets) offsets[j] = o;
-        o = align_up(o + gemv_partial_bytes(rows, (n_list[j] + COLS - 1) / COLS, p.n_kc), 256);
+        o = align_up(o + gemv_partial_bytes(rows, n_list[j] / GEMV_COLS, p.n_kc), 256);
     }
     if (plan) *plan = p;
     return o;
@@ -180,33 +209,29 @@ int exl3_gemm_group(const uint16_t* a, int64_t m, int64_t k, int64_t count, cons
         const int R = (int)(m - r0 < block ? m - r0 : block);
         FanParams P{};
         P.x = a + r0 * k;
-        P.R = R; P.K = (int)k; P.nsteps = p.nsteps; P.n_kc = p.n_kc; P.count = (int)count; P.out_kind = c_kind;
-        int blocks = 0, rblocks = 0;
-        bool whole = true;
+        P.R = R; P.K = (int)k; P.nsteps = p.nsteps; P.n_kc = p.n_kc; P.nkg = p.nkg; P.count = (int)count;
+        P.out_kind = c_kind; P.xcd = p.xcd ? 1 : 0;
+        int hbs = 0;
         for (int64_t j = 0; j < count; ++j) {
-            const int n_cb = (int)((n_list[j] + COLS - 1) / COLS);
             P.trellis[j] = trellis[j]; P.suh[j] = suh[j]; P.svh[j] = svh[j];
             P.out[j] = reinterpret_cast<char*>(c[j]) + (size_t)r0 * n_list[j] * c_elem;
             P.partials[j] = reinterpret_cast<float*>(reinterpret_cast<char*>(scratch) + offsets[j]);
             P.N[j] = (int)n_list[j];
             P.bits[j] = bits_list[j];
-            P.block0[j] = blocks;
-            P.rblock0[j] = rblocks;
-            blocks += n_cb * p.n_kc;
-            rblocks += (int)(n_list[j] / 128) * R;
-            whole = whole && n_list[j] % COLS == 0;
+            P.hb0[j] = hbs;
+            hbs += (int)(n_list[j] / GEMV_COLS);
         }
-        P.block0[count] = blocks;
-        P.rblock0[count] = rblocks;
-        P.xcd = xcd_order_allowed() && whole && (blocks / p.n_kc) % N_XCD == 0 ? 1 : 0;
+        P.hb0[count] = hbs;
         for (int b = 1; b <= 8; ++b) {
             if (!(widths & (1u << b))) continue;
             int rc = 0;
-            EXL3_BITS_SWITCH(b, rc = launch_gemv_fan<B_>(P, codebook, p.waves, blocks, s));
+            EXL3_BITS_SWITCH(b, rc = launch_gemv_fan<B_>(P, codebook, s));
             if (rc) return rc;
         }
-        hipLaunchKernelGGL(gemv_fan_reduce_kernel<RED_BATCH>, dim3(rblocks), dim3(64), 0, s, P);
-        if (int rc = check_launch()) return rc;
+        if (p.n_kc > 1) {
+            hipLaunchKernelGGL(gemv_fan_reduce_kernel<RED_BATCH>, dim3(hbs * R), dim3(64), 0, s, P);
+            if (int rc = check_launch()) return rc;
+        }
     }
     return 0;
 }

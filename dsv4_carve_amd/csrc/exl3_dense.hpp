@@ -4,6 +4,7 @@
 #pragma once
 
 #include <stdlib.h>
+#include <algorithm>
 
 #include "exl3_gemv.hpp"
 #include "exl3_capi_util.hpp"
@@ -274,368 +275,347 @@ __global__ __launch_bounds__(64) void had_rows_kernel(const void* x, int x_kind,
 
 // ---------------------------------------------------------------- dense GEMV
 //
-// An item is (256-column block cb, k-chunk kc of `nsteps` 64-row steps) of
-// y = had_in(x) . Wq for rows 0..R-1.  Its workgroup has W waves (1, 2 or 4):
-// wave w accumulates the output columns n in [w*16/W, (w+1)*16/W) of each of
-// the block's 16 n-tiles, so one step's decode is spread over W SIMDs with no
-// cross-wave sum.  Every wave loads the whole tile (a lane's windows interleave
-// the column groups); the repeats hit the CU's L1.  At few rows the call is
-// latency-bound: the plan shortens items and splits columns until there is a
-// wave per SIMD, so each wave decodes as little as possible.
+// y = had_in(x) . Wq for rows 0..R-1 (R <= 32), split over workgroups by
+// 128-column block (one output Hadamard block) and k-chunk.  A workgroup is
+// 2 x nkg waves (nkg = 2, 4 or 8): column half cg (64 columns, 4 n-tiles) and
+// k-group kg, which takes the chunk's 64-row steps kg, kg + nkg, ...  The
+// k-groups' sums meet in LDS, so a k-chunk of 512 rows leaves one partial
+// vector, and a call whose chunk is all of K is finished in the same launch.
+//
+// Quarter tiles.  Four lanes share an n-tile: lane c of a 16-lane row holds
+// columns n = 4j + p (p = c & 3) of n-tile c >> 2.  By the tile permutation
+// (tile_t) column n + p's windows sit 32 p elements after column n's for
+// n & 7 = 0 or 4, so the lane reads its tile rotated by p blocks of BITS words
+// and decodes columns 0, 4, 8 and 12 at their compile-time positions (the
+// stream is circular): 2 (BITS + 1) of the tile's 8 BITS words.  A step is
+// then 64 weights and 16 MFMAs per lane instead of 256 and 64, so a matrix of
+// a few million weights spreads over every SIMD with one short step per wave,
+// and each tile word is requested once instead of by every column group.
+// A few-row call is latency-bound: what this split shortens is the chain of
+// first load, rotation, decode and sum, and the partials that the finish reads
+// (one per 512 k-rows).  At 4096x4096, 6 bits, 1 row: input there at 1.2 us,
+// rotated 1.9, weights 2.45 (at memory rate), decoded and multiplied 4.7, sums
+// stored 5.5, plus two launches.  Against 256-column items of 128 k-rows on four
+// waves that each decode a quarter of every whole tile (us per call in a graph,
+// before / now): 4096x4096 6-bit 1 row 10.3 / 9.6, 16 rows 13.5 / 11.2, 32 rows
+// 18.2 / 14.5; 4096x1536 3-bit 16 rows 11.1 / 8.8; 4096x12288 4-bit 1 row 17.4 /
+// 15.2; 8192x8192 3-bit 16 rows 26.2 / 21.5; 2048x2048 2-bit 1 row 7.6 / 6.2.
+//
+// The rotated input is kept in LDS with every half doubled, so an MFMA's A
+// operand is one 16-byte read.
 
-constexpr int GEMV_NSTEP_CAP = 8;   // k rows per item <= 512
-constexpr int GEMV_MAX_WAVES = 4;   // column groups per item
+constexpr int GEMV_COLS = 128;      // columns per workgroup: one Hadamard block
+constexpr int GEMV_NCG = 2;         // column halves per workgroup
+constexpr int GEMV_MAX_NKG = 8;     // k-groups per workgroup
 constexpr int GEMV_MAX_ROWS = 32;   // rows per call: one or two 16-row MFMA blocks share each decode
+constexpr int GEMV_RED_LD = 130;    // row stride (floats) of the k-groups' sums in LDS
 
 struct GemvPlan {
-    int nsteps;         // steps (64 k-rows) per item
+    int nsteps;         // 64-row steps per k-chunk (even; the last chunk may hold fewer)
     int n_kc;           // k-chunks
-    int n_cb;           // 256-column blocks
-    int waves;          // waves per item (column groups), 1, 2 or 4
-    bool split_reduce;  // partial sums finished by gemv_reduce_kernel
+    int n_hb;           // 128-column blocks
+    int nkg;            // k-groups per workgroup
     bool xcd = false;   // items and finish keyed by column block (xcd_split)
 };
 
-// Rows of x per call of the kernels: up to 16 rows one MFMA row block, 17 and
-// more two (32 rows).
 inline int64_t gemv_block_rows(int64_t m) { return m > MAX_ROWS ? GEMV_MAX_ROWS : MAX_ROWS; }
 
-// EXL3_GEMV_STEPS / EXL3_GEMV_WAVES override the plan's steps per item
-// (1, 2, 4, 8; kept only if it divides the k steps) and waves per item
-// (1, 2, 4); EXL3_GEMV_LAST_ARRIVER=1 finishes every call in the last
-// arriving workgroup of each column block instead of a reduction launch.
-// 0 or unset: the plan below.
-inline int gemv_override(const char* name) {
-    const char* v = getenv(name);
+// EXL3_GEMV_STEPS overrides the plan's steps per k-chunk (an even number; read
+// at every call).
+inline int gemv_steps_override() {
+    const char* v = getenv("EXL3_GEMV_STEPS");
     const int x = v && *v ? atoi(v) : 0;
-    return (x == 1 || x == 2 || x == 4 || x == 8) ? x : 0;
+    return x >= 2 && x % 2 == 0 ? x : 0;
 }
 
-inline GemvPlan gemv_plan_cb(int64_t rows, int64_t k, int64_t total_cb, int cus) {
-    static const int env_steps = gemv_override("EXL3_GEMV_STEPS");
-    static const int env_waves = gemv_override("EXL3_GEMV_WAVES");
-    static const bool env_last = gemv_override("EXL3_GEMV_LAST_ARRIVER") == 1;
+// Rows of the A tile in LDS, odd so that the units of neighbouring k-slices
+// fall on different banks.
+__host__ __device__ constexpr int gemv_a_rows(int R) { return R | 1; }
+
+inline int gemv_lds_bytes(int64_t R, int nsteps, int nkg) {
+    const int64_t a = (int64_t)nsteps * 256 * gemv_a_rows((int)R);
+    const int64_t red = (int64_t)nkg * (R < MAX_ROWS ? R : MAX_ROWS) * GEMV_RED_LD * 4;
+    return (int)(a > red ? a : red);
+}
+
+inline GemvPlan gemv_plan_hb(int64_t rows, int64_t k, int64_t total_hb, int cus) {
+    const int env_steps = gemv_steps_override();
     GemvPlan p;
-    p.n_cb = (int)total_cb;
-    const int ksteps = (int)(k / STEP_K);
+    p.n_hb = (int)total_hb;
+    const int S = std::max((int)(k / STEP_K), 2);      // even
     const int64_t r = rows < GEMV_MAX_ROWS ? rows : GEMV_MAX_ROWS;
-    // Two waves per SIMD, with four column groups per item first: splitting
-    // columns costs nothing but repeated (L1-hit) tile loads, while shorter
-    // items cost fp32 partials (k-chunks x rows x 256 x 4 bytes per column
-    // block) and finish loads.  Measured at 1, 16, 32 and 144 rows on
-    // 4096x4096, 4096x1536, 1536x4096 and 4096x12288: four groups beat one
-    // and two at every shape, 2-step items beat 1-step ones, and the items
-    // this loop picks were the fastest or within 4% of them.
-    const int64_t target = 8LL * cus;
-    const int min_steps = 2;
-    int nsteps = GEMV_NSTEP_CAP;
-    while (nsteps > min_steps && total_cb * (ksteps / nsteps) * GEMV_MAX_WAVES < target) nsteps /= 2;
-    if (env_steps && ksteps % env_steps == 0) nsteps = env_steps;
-    while (ksteps % nsteps) nsteps /= 2;
-    const int64_t items = total_cb * (ksteps / nsteps);
-    int waves = GEMV_MAX_WAVES;
-    while (waves > 1 && items * (waves / 2) >= target) waves /= 2;
-    if (env_waves && env_waves <= GEMV_MAX_WAVES) waves = env_waves;
-    if (r > MAX_ROWS && waves < 2) waves = 2;    // 32-row blocks are built for 2 and 4 groups
+    const int cap = r > MAX_ROWS ? 16 : 32;            // LDS: at most 136 KB of A
+    // Chunk length by the time it is expected to take (us): rounds of
+    // workgroups a CU holds at once (16 waves), each a start of 2.7; the steps'
+    // decode at 0.43 per wave-step and SIMD, and their input's rotation; for a
+    // split K the finish launch, its loads and the partials' round trip.
+    // Against the best of 2-32 steps at 1, 4, 16 and 32 rows on nine shapes
+    // (512x256 to 8192x8192) the choice is within 4%.
+    int nsteps = 2;
+    double best = 1e30;
+    for (int ns = 2; ns <= cap && ns <= S; ns += 2) {
+        const int64_t n_kc = (S + ns - 1) / ns, wgs = total_hb * n_kc, per_cu = (wgs + cus - 1) / cus;
+        const int resident = ns >= 8 ? 1 : ns >= 4 ? 2 : 4;
+        double t = 2.7 * (double)((per_cu + resident - 1) / resident);
+        t += (double)(per_cu * ns) * (0.215 * (r > MAX_ROWS ? 1.3 : 1.0) + 0.0094 * (double)r);
+        if (n_kc > 1) t += 2.0 + 0.03 * (double)n_kc + 2e-6 * (double)(n_kc * r * total_hb * GEMV_COLS);
+        if (t < best) {
+            best = t;
+            nsteps = ns;
+        }
+    }
+    if (env_steps && env_steps <= cap) nsteps = env_steps < S ? env_steps : S;
     p.nsteps = nsteps;
-    p.n_kc = ksteps / nsteps;
-    p.waves = waves;
-    // The last arriver of a 256-column block would sum rows * n_kc partial
-    // vectors behind a device-scope counter; beyond a handful, a separate
-    // reduction launch is shorter.
-    p.split_reduce = r * p.n_kc > 4 && !env_last;
+    p.n_kc = (S + nsteps - 1) / nsteps;
+    p.nkg = nsteps >= 8 ? 8 : nsteps >= 4 ? 4 : 2;
     return p;
 }
 
-// The partial-sum items of a column block and that block's finish run on one
-// XCD (xcd_split) when the column blocks (of a matrix, or of all members of a
-// fan) are whole and a multiple of 8: 16 rows of 4096x4096 14.0 against 16.0
-// us, the gain in the partial-sum launch.  EXL3_XCD_ORDER=0 turns it off (read
-// at every call, so one process can compare both orders).
+// The items of a column block and that block's finish run on one XCD
+// (xcd_split) when the column blocks (of a matrix, or of all members of a fan)
+// are a multiple of 8.  EXL3_XCD_ORDER=0 turns it off (read at every call, so
+// one process can compare both orders).
 inline bool xcd_order_allowed() {
     const char* v = getenv("EXL3_XCD_ORDER");
     return !(v && *v && atoi(v) == 0);
 }
 
 inline GemvPlan gemv_plan(int64_t rows, int64_t k, int64_t n, int cus) {
-    GemvPlan p = gemv_plan_cb(rows, k, (n + COLS - 1) / COLS, cus);
-    p.xcd = xcd_order_allowed() && n % COLS == 0 && p.n_cb % N_XCD == 0;
+    GemvPlan p = gemv_plan_hb(rows, k, std::max<int64_t>(n / GEMV_COLS, 1), cus);
+    p.xcd = xcd_order_allowed() && p.n_hb % N_XCD == 0;
     return p;
 }
 
-// Split-K partials of a matrix: [column block][row][k-chunk][256] fp32, so
+// Split-K partials of a matrix: [128-column block][row][k-chunk][128] fp32, so
 // the finish of one (column block, row) reads its k-chunks from one
 // contiguous range (strided reads of the same offset in every k-chunk all
 // fell on a few memory channels).
-inline int64_t gemv_partial_bytes(int64_t rows, int64_t n_cb, int64_t n_kc) {
-    return n_cb * (rows < GEMV_MAX_ROWS ? rows : GEMV_MAX_ROWS) * n_kc * COLS * 4;
+inline int64_t gemv_partial_bytes(int64_t rows, int64_t n_hb, int64_t n_kc) {
+    return n_kc > 1 ? n_hb * (rows < GEMV_MAX_ROWS ? rows : GEMV_MAX_ROWS) * n_kc * GEMV_COLS * 4 : 0;
 }
-__device__ __forceinline__ size_t gemv_partial_off(int cb, int row, int kc, int R, int n_kc) {
-    return ((size_t)(cb * R + row) * n_kc + kc) * COLS;
-}
-
-inline int64_t gemv_scratch_bytes(int64_t rows, int64_t k, int64_t n, int cus) {
-    const GemvPlan p = gemv_plan(rows, k, n, cus);
-    const int64_t ctr = align_up((int64_t)p.n_cb * 4, 256);
-    return ctr + gemv_partial_bytes(rows, p.n_cb, p.n_kc);
+__device__ __forceinline__ size_t gemv_partial_off(int hb, int row, int kc, int R, int n_kc) {
+    return ((size_t)(hb * R + row) * n_kc + kc) * GEMV_COLS;
 }
 
-// Input rotation of one item: rows 0..R-1, k in [k0, k0 + span), into the LDS
-// A tile, by the item's W waves.  A job is (row, 128-block); for a 64-row
-// item the block is rotated whole and its other half dropped.  A batch's
-// loads are all issued before its arithmetic.
-constexpr int ROT_BATCH = 16;
+// 8 consecutive halves at any 2-byte alignment, as one 16-byte load where the
+// target allows it.
+__device__ __forceinline__ u32x4_t load_half8(const uint16_t* p) {
+    typedef u32x4_t __attribute__((aligned(2))) u32x4_u;
+    return *(gptr_t<u32x4_u>)p;
+}
 
-struct RotJobs {
-    int kb0, nblk, jobs, span;
-};
-struct RotBatch {
-    uint32_t x[ROT_BATCH], s[ROT_BATCH];
+// The words of a lane's quarter tile: rotated blocks 0 and 4 and the word
+// before each (the windows of columns 0, 4, 8 and 12 reach at most 16 - BITS
+// bits back).  The other words are never written or read, so they take no
+// registers.
+template <int BITS>
+struct QuarterTile {
+    uint32_t w[8 * BITS];
 };
 
-__device__ __forceinline__ RotJobs rot_jobs(int k0, int nsteps, int R) {
-    RotJobs j;
-    j.span = nsteps * STEP_K;
-    j.kb0 = k0 & ~127;
-    j.nblk = (k0 + j.span - j.kb0 + 127) >> 7;
-    j.jobs = R * j.nblk;
-    return j;
-}
-
-__device__ __forceinline__ void rot_load(const uint16_t* x, int K, const uint16_t* suh, const RotJobs& J, int j0,
-                                         int stride, RotBatch& b) {
-    const int lane = threadIdx.x & (WAVE - 1);
-#pragma unroll
-    for (int i = 0; i < ROT_BATCH; ++i) {
-        const int j = j0 + i * stride;
-        if (j < J.jobs) {
-            const int m = j / J.nblk, blk = j - m * J.nblk;
-            const int kk = J.kb0 + 128 * blk + 2 * lane;
-            b.x[i] = *reinterpret_cast<const uint32_t*>(x + (size_t)m * K + kk);
-            b.s[i] = *reinterpret_cast<const uint32_t*>(suh + kk);
-        }
+template <int N>
+__device__ __forceinline__ void load_words_g(uint32_t* dst, gptr_t<uint32_t> src) {
+    typedef u32x4_t __attribute__((aligned(4))) u32x4_u;
+    typedef uint32_t u32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+    if constexpr (N >= 4) {
+        const u32x4_t v = *(gptr_t<u32x4_u>)src;
+        dst[0] = v[0]; dst[1] = v[1]; dst[2] = v[2]; dst[3] = v[3];
+        if constexpr (N > 4) load_words_g<N - 4>(dst + 4, src + 4);
+    } else if constexpr (N >= 2) {
+        const u32x2_u v = *(gptr_t<u32x2_u>)src;
+        dst[0] = v[0]; dst[1] = v[1];
+        if constexpr (N > 2) dst[2] = src[2];
+    } else {
+        dst[0] = src[0];
     }
 }
 
-__device__ __forceinline__ void rot_store(const RotJobs& J, int k0, int j0, int stride, const RotBatch& b,
-                                          uint16_t* xa) {
-    const int lane = threadIdx.x & (WAVE - 1);
-#pragma unroll
-    for (int i = 0; i < ROT_BATCH; ++i) {
-        const int j = j0 + i * stride;
-        if (j < J.jobs) {
-            const int m = j / J.nblk, blk = j - m * J.nblk;
-            const uint32_t h = had_in_pair(b.x[i], b.s[i], 0);
-            const int kr = J.kb0 + 128 * blk + 2 * lane - k0;   // even: both halves in one step
-            if (kr >= 0 && kr < J.span) {
-                xa[xa_index(m, kr >> 6, GEMV_NSTEP_CAP, kr & 63)] = (uint16_t)(h & 0xffffu);
-                xa[xa_index(m, kr >> 6, GEMV_NSTEP_CAP, (kr & 63) + 1)] = (uint16_t)(h >> 16);
-            }
-        }
-    }
+// `t`: the lane's tile (8 BITS words), p: its rotation in blocks of BITS words.
+template <int BITS>
+__device__ __forceinline__ void load_quarter(QuarterTile<BITS>& d, gptr_t<uint32_t> t, int p) {
+    load_words_g<BITS>(d.w, t + p * BITS);
+    d.w[8 * BITS - 1] = t[p ? p * BITS - 1 : 8 * BITS - 1];
+    load_words_g<BITS + 1>(d.w + 4 * BITS - 1, t + (p + 4) * BITS - 1);
 }
 
-// Decodes output columns [N0, N0+NC) of each n-tile of the lane's tile and
-// accumulates them into each of the RB 16-row blocks (acc[rb][j] = column
-// N0 + j); the MFMA sequence per column and row block is the one mma_tile
-// issues.
-template <int BITS, int CB, int N0, int NC, int RB>
-__device__ __forceinline__ void mma_tile_cols(const uint32_t* W, const half8_t (&A)[RB][4],
-                                              float4_t (&acc)[RB][NC]) {
-    static_for<NC>([&](auto JI) {
-        constexpr int j = decltype(JI)::value;
-        constexpr int n = N0 + j;
-        static_for<4>([&](auto RI) {
-            constexpr int r = decltype(RI)::value;
-            constexpr int T0 = 32 * (n & 7) + 8 * r + 4 * (n >> 3);
-            u32x4_t b;
-            b[0] = decode_pair<BITS, CB, T0 + 0>(W);
-            b[1] = decode_pair<BITS, CB, T0 + 1>(W);
-            b[2] = decode_pair<BITS, CB, T0 + 2>(W);
-            b[3] = decode_pair<BITS, CB, T0 + 3>(W);
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-                acc[rb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[rb][r], __builtin_bit_cast(half8_t, b),
-                                                                     acc[rb][j], 0, 0, 0);
-        });
-    });
+// The lane's MFMA columns in decode order: columns n and n + 8, whose eight
+// windows at one k-group are consecutive in the stream, back to back.
+__host__ __device__ constexpr int quarter_col(int j) { return 4 * (j >> 1) + 8 * (j & 1); }
+
+// Output rotation, svh and store of two consecutive columns per lane of one
+// row's 128-column block.
+__device__ __forceinline__ void gemv_finish(float v0, float v1, const uint16_t* __restrict__ svh,
+                                            void* __restrict__ out, int out_kind, int N, int row, int col) {
+    const float w0 = f16_bits_to_f32(svh[col]), w1 = f16_bits_to_f32(svh[col + 1]);
+    fwht128_x2(v0, v1);
+    store_out(out, (size_t)row * N + col, out_kind, v0 * HAD_NORM * w0);
+    store_out(out, (size_t)row * N + col + 1, out_kind, v1 * HAD_NORM * w1);
 }
 
-// The item's `nsteps` steps (any count >= 1) for columns [N0, N0+NC).  `first`
-// holds step 0's tile (loaded by the caller); later tiles are loaded one step
-// ahead.  The load two steps on sits behind a branch, unlike mma_steps: the
-// short dense items then keep 2 waves per SIMD resident.
-template <int BITS, int CB, int N0, int NC, int RB>
-__device__ __forceinline__ void gemv_mma(TileRegs<BITS>& first, const u32x4_t* p, int n16, int nsteps, int R,
-                                         const uint16_t* xa, float4_t (&acc)[RB][NC]) {
+// One item: 128-column block hb, k-chunk kc.  smem: gemv_lds_bytes.
+template <int BITS, int CB, int RB>
+__device__ __forceinline__ void gemv_item(const uint16_t* __restrict__ x, const int16_t* __restrict__ trellis,
+                                          const uint16_t* __restrict__ suh, const uint16_t* __restrict__ svh,
+                                          void* __restrict__ out, int out_kind, int R, int K, int N, int nsteps,
+                                          int n_kc, int hb, int kc, float* __restrict__ partials, char* smem) {
     const int lane = threadIdx.x & (WAVE - 1);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int nw = (int)blockDim.x / WAVE, nkg = nw / GEMV_NCG;
+    const int cg = w & (GEMV_NCG - 1), kg = w / GEMV_NCG;
     const int g = lane >> 4, c = lane & 15;
-    const size_t step = (size_t)4 * n16 * tile_vecs<BITS>();
-    // A rows >= R repeat row R-1 (a valid row, no branch): their outputs are never stored
-    int arow[RB];
+    const int s0 = kc * nsteps, ns = min(nsteps, K / STEP_K - s0);     // this chunk's steps, even
+    const int Rp = gemv_a_rows(R);
+
+    // Input rotation jobs: (row, 128-block), one per 16 lanes.  The first
+    // pass's inputs are requested before the weights, so waiting for them
+    // (loads complete in issue order) does not wait for the tile.
+    const int nblk = ns / 2, jobs = R * nblk;
+    u32x4_t xv, sv;
+    int row, blk;
+    auto rot_load = [&](int j0) {
+        const int id = min(j0 + g, jobs - 1);
+        row = id / nblk;
+        blk = id - row * nblk;
+        const int col = s0 * STEP_K + 128 * blk + 8 * c;
+        xv = load_half8(x + (size_t)row * K + col);
+        sv = load_half8(suh + col);
+    };
+    if (4 * w < jobs) rot_load(4 * w);
+
+    // the lane's quarter tile of step s
+    const int p = c & 3, n16 = N / 16;
+    gptr_t<uint32_t> tp = as_global(reinterpret_cast<const uint32_t*>(trellis)) +
+                          ((size_t)(4 * (s0 + kg) + g) * n16 + 8 * hb + 4 * cg + (c >> 2)) * (8 * BITS);
+    const size_t tstep = (size_t)4 * nkg * n16 * (8 * BITS);
+    QuarterTile<BITS> t0, t1;
+    if (kg < ns) load_quarter<BITS>(t0, tp, p);
+
+    for (int j0 = 4 * w; j0 < jobs; j0 += 4 * nw) {
+        if (j0 != 4 * w) rot_load(j0);
+        float v[8];
+        scaled8(xv, sv, 0, v);
+        const u32x4_t h = rotated8(v);
+        if (j0 + g < jobs) {
+            // halves 8c .. 8c + 7 of the block: k-slice c >> 1, its lower or upper 8 rows;
+            // k-group r takes rows 2r, 2r + 1 of both (unit [slice][r][row], 16 bytes)
+            uint2* d = reinterpret_cast<uint2*>(smem) + (size_t)((8 * blk + (c >> 1)) * 4 * Rp + row) * 2 + (c & 1);
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) arow[rb] = min(16 * rb + c, R - 1);
+            for (int r = 0; r < 4; ++r)
+                d[(size_t)r * Rp * 2] = make_uint2(__builtin_amdgcn_perm(h[r], h[r], 0x01000100u),
+                                                   __builtin_amdgcn_perm(h[r], h[r], 0x03020302u));
+        }
+    }
+    __syncthreads();
+
+    float4_t acc[RB][4];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int i = 0; i < NC; ++i) acc[rb][i] = float4_t{0.f, 0.f, 0.f, 0.f};
-    auto step_mma = [&](const TileRegs<BITS>& t, int si) {
+        for (int j = 0; j < 4; ++j) acc[rb][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    // A rows >= R repeat row R-1 (a valid row, no branch): their outputs are never stored
+    const half8_t* ap[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+        ap[rb] = reinterpret_cast<const half8_t*>(smem) + g * 4 * Rp + min(16 * rb + c, R - 1);
+
+    auto step_mma = [&](const QuarterTile<BITS>& t, int s) {
         half8_t A[RB][4];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) A[rb][r] = a_operand(xa, arow[rb], si, GEMV_NSTEP_CAP, g, r);
-        mma_tile_cols<BITS, CB, N0, NC, RB>(t.words(), A, acc);
+            for (int r = 0; r < 4; ++r) A[rb][r] = ap[rb][(16 * s + r) * Rp];
+        static_for<4>([&](auto JI) {
+            constexpr int j = decltype(JI)::value, n = quarter_col(j);
+            static_for<4>([&](auto RI) {
+                constexpr int r = decltype(RI)::value;
+                constexpr int T0 = 32 * (n & 7) + 8 * r + 4 * (n >> 3);
+                u32x4_t b;
+                b[0] = decode_pair<BITS, CB, T0 + 0>(t.w);
+                b[1] = decode_pair<BITS, CB, T0 + 1>(t.w);
+                b[2] = decode_pair<BITS, CB, T0 + 2>(t.w);
+                b[3] = decode_pair<BITS, CB, T0 + 3>(t.w);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+                    acc[rb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[rb][r], __builtin_bit_cast(half8_t, b),
+                                                                        acc[rb][j], 0, 0, 0);
+            });
+        });
     };
-    TileRegs<BITS> second;
-    int s = 0;
-    for (; s + 1 < nsteps; s += 2) {
-        load_tile<BITS>(second, p + (s + 1) * step);
-        step_mma(first, s);
-        if (s + 2 < nsteps) load_tile<BITS>(first, p + (s + 2) * step);
-        step_mma(second, s + 1);
-    }
-    if (nsteps & 1) step_mma(first, s);
-}
-
-// One item by its W waves: fp32 partial sums of rows < R stored to the
-// partials at gemv_partial_off(cb, row, kc) (DEV: device-scope stores, read in the same launch;
-// otherwise plain stores, read by a later launch).  xa: the item's LDS.
-template <int BITS, int CB, int W, int RB, bool DEV>
-__device__ __forceinline__ void gemv_item(const uint16_t* __restrict__ x, const int16_t* __restrict__ trellis,
-                                          const uint16_t* __restrict__ suh, int R, int K, int N, int nsteps, int cb,
-                                          int kc, float* __restrict__ partials, uint16_t* xa) {
-    constexpr int NC = 16 / W;
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
-    const int k0 = kc * nsteps * STEP_K;
-    const u32x4_t* tp = tile_ptr<BITS>(trellis, N / 16, k0 / 16, cb * 16);
-
-    // first rotation batch's loads, then step 0's tile, then the rotation
-    const RotJobs J = rot_jobs(k0, nsteps, R);
-    RotBatch rb;
-    rot_load(x, K, suh, J, w, W, rb);
-    TileRegs<BITS> first;
-    load_tile<BITS>(first, tp);
-    rot_store(J, k0, w, W, rb, xa);
-    for (int j0 = w + W * ROT_BATCH; j0 < J.jobs; j0 += W * ROT_BATCH) {
-        rot_load(x, K, suh, J, j0, W, rb);
-        rot_store(J, k0, j0, W, rb, xa);
-    }
-    __syncthreads();
-
-    float4_t acc[RB][NC];
-    if constexpr (W == 1) {
-        gemv_mma<BITS, CB, 0, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
-    } else if constexpr (W == 2) {
-        if (w == 0) gemv_mma<BITS, CB, 0, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
-        else gemv_mma<BITS, CB, NC, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
-    } else {
-        static_assert(W == 4, "1, 2 or 4 waves per item");
-        if (w == 0) gemv_mma<BITS, CB, 0, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
-        else if (w == 1) gemv_mma<BITS, CB, NC, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
-        else if (w == 2) gemv_mma<BITS, CB, 2 * NC, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
-        else gemv_mma<BITS, CB, 3 * NC, NC, RB>(first, tp, N / 16, nsteps, R, xa, acc);
+    for (int s = kg; s < ns; s += 2 * nkg) {
+        if (s + nkg < ns) load_quarter<BITS>(t1, tp + tstep, p);
+        step_mma(t0, s);
+        if (s + nkg < ns) {
+            tp += 2 * tstep;
+            if (s + 2 * nkg < ns) load_quarter<BITS>(t0, tp, p);
+            step_mma(t1, s + nkg);
+        }
     }
 
-    // Transpose through LDS (the A tile is free once every wave is past its
-    // MFMAs) so each store instruction writes one contiguous 1 KB row.
-    __syncthreads();
-    float* tbuf = reinterpret_cast<float*>(xa);
-    {
-        const int c = lane & 15, rg = lane >> 4;
+    // Sum over the k-groups in LDS, one 16-row block at a time, then the
+    // finish (whole K) or the chunk's partial vector.
+    float* red = reinterpret_cast<float*>(smem);
+    const int hcol = 128 * hb + 2 * lane;
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
+    for (int rb = 0; rb < RB; ++rb) {
+        const int rows = min(R - 16 * rb, 16);
+        __syncthreads();                               // A (or the previous block's sums) no longer read
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = 16 * rb + 4 * rg + i;
-                if (row < R) {
-                    float4_t* t = reinterpret_cast<float4_t*>(tbuf + row * COLS + 16 * c + w * NC);
+        for (int i = 0; i < 4; ++i) {
+            const int m = 4 * g + i;
+            if (m < rows) {
+                float* d = red + (size_t)(kg * min(R, 16) + m) * GEMV_RED_LD + 64 * cg + 16 * (c >> 2) + p;
 #pragma unroll
-                    for (int q = 0; q < NC / 4; ++q)
-                        t[q] = float4_t{acc[rb][4 * q][i], acc[rb][4 * q + 1][i], acc[rb][4 * q + 2][i],
-                                        acc[rb][4 * q + 3][i]};
-                }
+                for (int j = 0; j < 4; ++j) d[quarter_col(j)] = acc[rb][j][i];
             }
-    }
-    __syncthreads();
-    const int cols = min(COLS, N - cb * COLS);
-    const int n_kc = K / (nsteps * STEP_K);
-    if (4 * lane < cols)
-        for (int row = w; row < R; row += W) {
-            const float4_t v = reinterpret_cast<const float4_t*>(tbuf + row * COLS)[lane];
-            float* d = partials + gemv_partial_off(cb, row, kc, R, n_kc) + 4 * lane;
-            if constexpr (DEV) st_dev4(d, v);
-            else *reinterpret_cast<float4_t*>(d) = v;
         }
+        __syncthreads();
+        for (int m = w; m < rows; m += nw) {
+            float v0 = 0.f, v1 = 0.f;
+#pragma unroll
+            for (int q = 0; q < GEMV_MAX_NKG; ++q)
+                if (q < nkg) {
+                    const float2 t = *reinterpret_cast<const float2*>(red + (size_t)(q * min(R, 16) + m) * GEMV_RED_LD + 2 * lane);
+                    v0 += t.x;
+                    v1 += t.y;
+                }
+            if (n_kc > 1)
+                *reinterpret_cast<float2*>(partials + gemv_partial_off(hb, 16 * rb + m, kc, R, n_kc) + 2 * lane) =
+                    make_float2(v0, v1);
+            else
+                gemv_finish(v0, v1, svh, out, out_kind, N, 16 * rb + m, hcol);
+        }
+    }
 }
 
-// SPLIT: store the partials and stop (gemv_reduce_kernel finishes them);
-// otherwise the last arriver of each column block finishes it (wave 0).
-template <int BITS, int CB, int W, int RB, bool SPLIT>
-__global__ __launch_bounds__(64 * W) void gemv_kernel(const uint16_t* __restrict__ x,
-                                                      const int16_t* __restrict__ trellis,
-                                                      const uint16_t* __restrict__ suh,
-                                                      const uint16_t* __restrict__ svh, void* __restrict__ out,
-                                                      int out_kind, int R, int K, int N, int nsteps, int n_kc,
-                                                      int xcd, int* __restrict__ counters,
-                                                      float* __restrict__ partials) {
-    __shared__ uint16_t xa[MAX_ROWS * RB * GEMV_NSTEP_CAP * STEP_K];
-    int cb, kc;
-    xcd_split(blockIdx.x, n_kc, xcd, cb, kc);      // group: column block
-    gemv_item<BITS, CB, W, RB, !SPLIT>(x, trellis, suh, R, K, N, nsteps, cb, kc, partials, xa);
-    if constexpr (SPLIT) return;
-    publish_fence();
-    __syncthreads();
-    if (threadIdx.x >= WAVE) return;
-    const int lane = threadIdx.x;
-    int old = 0;
-    if (lane == 0) old = atomicAdd(&counters[cb], 1);
-    old = __shfl(old, 0, 64);
-    if (old != n_kc - 1) return;
-
-    // Last arriver: fixed-order split-K sum, output Hadamard, svh, store.
-    const int col = cb * COLS + 128 * (lane >> 5) + 4 * (lane & 31);
-    const bool ok = col < N;
-    float sv[4] = {0.f, 0.f, 0.f, 0.f};
-    if (ok)
-        for (int e = 0; e < 4; ++e) sv[e] = f16_bits_to_f32(svh[col + e]);
-    for (int m = 0; m < R; ++m) {
-        float v[4] = {0.f, 0.f, 0.f, 0.f};
-        if (ok) {
-            const float4_t t = sum_partials(partials + gemv_partial_off(cb, m, 0, R, n_kc),
-                                            (uint32_t)(col - cb * COLS) * 4u, (size_t)COLS, n_kc);
-            v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
-        }
-        fwht128_x4(v);
-        if (ok)
-            for (int e = 0; e < 4; ++e) store_out(out, (size_t)m * N + col + e, out_kind, v[e] * HAD_NORM * sv[e]);
-    }
-    if (lane == 0) __hip_atomic_store(&counters[cb], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+template <int BITS, int CB, int RB>
+__global__ __launch_bounds__(WAVE * GEMV_NCG * GEMV_MAX_NKG) void gemv_kernel(
+    const uint16_t* __restrict__ x, const int16_t* __restrict__ trellis, const uint16_t* __restrict__ suh,
+    const uint16_t* __restrict__ svh, void* __restrict__ out, int out_kind, int R, int K, int N, int nsteps, int n_kc,
+    int xcd, float* __restrict__ partials) {
+    extern __shared__ __align__(16) char gemv_smem[];
+    int hb, kc;
+    xcd_split(blockIdx.x, n_kc, xcd, hb, kc);          // group: column block
+    gemv_item<BITS, CB, RB>(x, trellis, suh, svh, out, out_kind, R, K, N, nsteps, n_kc, hb, kc, partials, gemv_smem);
 }
 
 // Split-K finish of (128-column block hb, row m): the partials of chunks
-// 0..n_kc-1 summed in chunk order (as the last-arriver path does), output
-// Hadamard, svh, store; two columns per lane, up to RED_BATCH loads in
-// flight.  Plain loads: a previous launch wrote the partials.
-constexpr int RED_BATCH = 64;
+// 0..n_kc-1 summed in chunk order, output Hadamard, svh, store; two columns
+// per lane, up to RED_BATCH loads in flight.  Plain loads: a previous launch
+// wrote the partials.
+constexpr int RED_BATCH = 16;
 
 template <int BATCH>
 __device__ __forceinline__ void gemv_reduce_block(const float* __restrict__ partials, const uint16_t* __restrict__ svh,
                                                   void* __restrict__ out, int out_kind, int R, int N, int n_kc,
                                                   int hb, int m) {
     const int lane = threadIdx.x & (WAVE - 1);
-    const int col = hb * 128 + 2 * lane;
-    const uint32_t s2 = *reinterpret_cast<const uint32_t*>(svh + col);
-    const int cb = hb >> 1;
-    const float* p = partials + gemv_partial_off(cb, m, 0, R, n_kc) + (col - cb * COLS);
-    const size_t stride = COLS;
+    const float* p = partials + gemv_partial_off(hb, m, 0, R, n_kc) + 2 * lane;
     float v0 = 0.f, v1 = 0.f;
     for (int k0 = 0; k0 < n_kc; k0 += BATCH) {
         float2 t[BATCH];
 #pragma unroll
         for (int j = 0; j < BATCH; ++j)
-            if (k0 + j < n_kc) t[j] = *reinterpret_cast<const float2*>(p + (size_t)(k0 + j) * stride);
+            if (k0 + j < n_kc) t[j] = *reinterpret_cast<const float2*>(p + (size_t)(k0 + j) * GEMV_COLS);
 #pragma unroll
         for (int j = 0; j < BATCH; ++j)
             if (k0 + j < n_kc) {
@@ -643,23 +623,354 @@ __device__ __forceinline__ void gemv_reduce_block(const float* __restrict__ part
                 v1 = v1 + t[j].y;
             }
     }
-    fwht128_x2(v0, v1);
-    store_out(out, (size_t)m * N + col, out_kind, v0 * HAD_NORM * f16_bits_to_f32(s2 & 0xffffu));
-    store_out(out, (size_t)m * N + col + 1, out_kind, v1 * HAD_NORM * f16_bits_to_f32(s2 >> 16));
+    gemv_finish(v0, v1, svh, out, out_kind, N, m, 128 * hb + 2 * lane);
 }
 
 // Split-K finish, one wave per (128-column block, row).  Runs after
-// gemv_kernel<.., true> on the same stream.
+// gemv_kernel on the same stream.
 template <int BATCH>
 __global__ __launch_bounds__(64) void gemv_reduce_kernel(const float* __restrict__ partials,
                                                          const uint16_t* __restrict__ svh, void* __restrict__ out,
                                                          int out_kind, int R, int N, int n_kc, int xcd) {
-    // group: the 256-column block (two 128-blocks) whose partials gemv_kernel wrote on this XCD
-    int cb, j;
-    xcd_split(blockIdx.x, 2 * R, xcd, cb, j);
-    const int hi = j >= R ? 1 : 0;
-    const int hb = 2 * cb + hi, m = j - hi * R;
+    int hb, m;
+    xcd_split(blockIdx.x, R, xcd, hb, m);              // group: the block whose partials were written on this XCD
     gemv_reduce_block<BATCH>(partials, svh, out, out_kind, R, N, n_kc, hb, m);
+}
+
+// ---------------------------------------------------------------- dense GEMM (33 to a few hundred rows)
+//
+// y = xh . Wq for rows in tiles of 16 RB (RB <= 5) rows, as the GEMV above but
+// with the rotation in a launch of its own (its cost per column block would
+// grow with the rows): gemm_rotate_kernel writes had_in(x) with every half
+// doubled, in units of 16 bytes [step][k-slice][k-group][row], so the A
+// operand of an MFMA is one coalesced 16-byte load per lane (from L2: the
+// rotated input is 4 K bytes a row).  Each decoded operand feeds RB row
+// blocks.  A workgroup is GEMM_NKG k-groups of a (64-column half of a
+// 128-column block, k-chunk, row tile); their sums meet in LDS and leave one
+// partial tile in the accumulators' own layout, which gemm_finish_kernel sums
+// over the k-chunks, rotates and stores.  A chunk of the k-groups' length keeps
+// the partials short: they are written, flushed at the launch's end and read
+// again, and cost more than the decode (72 rows of 4096x4096 at 4 bits, of
+// 11.5 us: first loads 1.4, decode and MFMAs 4.5, exchange and store 1.5, the
+// rest launch and flush).
+//
+// What it replaces above 32 rows is the reconstructed weight in memory and a
+// library GEMM between two row-Hadamard launches.  Us per call, before / with
+// this kernel (bf16 out): 4096x4096 at 4 bits, 33 rows 31.7 / 16.9, 72 rows
+// 34.9 / 20.1, 128 rows 40.4 / 23.3, 256 rows 40.3 / 34.0; 4096x12288 at 6
+// bits, 72 rows 65.8 / 32.2, 256 rows 89.4 / 73.2; 1536x4096 at 3 bits, 256
+// rows 28.9 / 19.8.  From 384 rows the reconstructed weight is read often
+// enough to win (4096x4096 44.1 / 48, 512 rows 49.4 / 64.5).
+
+constexpr int GEMM_NKG = 8;
+constexpr int GEMM_MAX_RB = 5;      // LDS of the k-groups' exchange: 28 KB per row block
+
+// Rows of one GEMM launch (exl3_gemm runs more rows in slabs of this many).
+constexpr int GEMM_MAX_ROWS = 256;
+
+// Rows that take this path: above 32 all, 17-32 where the columns are many
+// enough that rotating the rows in every column block's workgroups costs more
+// than a launch (32 rows, GEMV / GEMM us: 4096x12288 35 / 26, 8192x8192 35 /
+// 27, but 4096x4096 14.5 / 17).
+// The rotated input's byte offsets are 32-bit.
+inline bool gemm_takes(int64_t m, int64_t k, int64_t n) {
+    return k <= (1 << 20) && (m > GEMV_MAX_ROWS || (m > MAX_ROWS && n >= 8192));
+}
+
+struct GemmPlan {
+    int rb;             // 16-row blocks per row tile
+    int n_rt;           // row tiles
+    int nsteps, n_kc;   // 64-row steps per k-chunk (the last may hold fewer), k-chunks
+    int n_hb;           // 128-column blocks
+    int64_t xd_bytes, partial_bytes;
+};
+
+inline GemmPlan gemm_plan(int64_t R, int64_t k, int64_t n, int cus) {
+    GemmPlan p;
+    p.n_hb = std::max((int)(n / GEMV_COLS), 1);
+    p.n_rt = (int)((R + 16 * GEMM_MAX_RB - 1) / (16 * GEMM_MAX_RB));
+    const int rows = (int)((R + p.n_rt - 1) / p.n_rt);
+    p.rb = (rows + 15) / 16;
+    if (p.rb < 2) p.rb = 2;
+    const int S = std::max((int)(k / STEP_K), 1);
+    // k-chunks: whole rounds of one workgroup per CU, each a start (us) and a
+    // step's decode and MFMAs per step of a wave (two waves a SIMD), plus the
+    // partials' way to memory and back.  On 4096x4096, 4096x12288, 1536x4096,
+    // 8192x8192 and 2048x512 at 33-512 rows the count this picks is within 3%
+    // of the best of 1, 2, 3, 4, 6 and 8.
+    const double ts = 0.75 + 0.13 * p.rb;
+    double best = 1e30;
+    for (int kc = 1; kc <= 32 && kc <= S; ++kc) {
+        const int ns = (S + kc - 1) / kc, n_kc = (S + ns - 1) / ns;
+        if (n_kc != kc) continue;
+        const int64_t wgs = (int64_t)p.n_hb * GEMV_NCG * p.n_rt * n_kc;
+        const double rounds = (double)((wgs + cus - 1) / cus);
+        const double t = rounds * (1.5 + ts * ((ns + GEMM_NKG - 1) / GEMM_NKG)) + 2e-6 * n_kc * (double)R * (double)n;
+        if (t < best) {
+            best = t;
+            p.nsteps = ns;
+            p.n_kc = n_kc;
+        }
+    }
+    const int64_t Rp = (int64_t)p.n_rt * 16 * p.rb;
+    p.xd_bytes = Rp * k * 4;
+    p.partial_bytes = (int64_t)p.n_hb * p.n_kc * Rp * GEMV_COLS * 4;
+    return p;
+}
+
+// Scratch of exactly this call.
+inline int64_t dense_scratch_bytes(int64_t rows, int64_t k, int64_t n, int cus) {
+    if (!gemm_takes(rows, k, n)) {
+        const GemvPlan p = gemv_plan(rows, k, n, cus);
+        return align_up(gemv_partial_bytes(rows, p.n_hb, p.n_kc), 256) + 256;
+    }
+    const GemmPlan g = gemm_plan(rows < GEMM_MAX_ROWS ? rows : GEMM_MAX_ROWS, k, n, cus);
+    int64_t b = align_up(g.xd_bytes, 256) + g.partial_bytes;
+    if (rows > GEMM_MAX_ROWS && rows % GEMM_MAX_ROWS)
+        b = std::max(b, dense_scratch_bytes(rows % GEMM_MAX_ROWS, k, n, cus));      // the last slab
+    return b;
+}
+
+template <int DUMMY = 0>
+__global__ __launch_bounds__(256) void gemm_rotate_kernel(const uint16_t* __restrict__ x,
+                                                          const uint16_t* __restrict__ suh, int R, int K, int Rp,
+                                                          u32x4_t* __restrict__ xd) {
+    // one wave: four rows of one 128-block
+    const int lane = threadIdx.x & (WAVE - 1), c = lane & 15;
+    const int nblk = K / 128;
+    const int id = (int)blockIdx.x * 4 + (int)(threadIdx.x / WAVE);
+    const int rg = id / nblk, blk = id - rg * nblk;
+    const int row = 4 * rg + (lane >> 4);
+    if (4 * rg >= R) return;
+    const int rr = min(row, R - 1);
+    const int col = 128 * blk + 8 * c;
+    const u32x4_t xv = load_half8(x + (size_t)rr * K + col), sv = load_half8(suh + col);
+    float v[8];
+    scaled8(xv, sv, 0, v);
+    const u32x4_t h = rotated8(v);
+    if (row >= R) return;
+    uint2* d = reinterpret_cast<uint2*>(xd) + ((size_t)(8 * blk + (c >> 1)) * 4 * Rp + row) * 2 + (c & 1);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        d[(size_t)r * Rp * 2] = make_uint2(__builtin_amdgcn_perm(h[r], h[r], 0x01000100u),
+                                           __builtin_amdgcn_perm(h[r], h[r], 0x03020302u));
+}
+
+// Partial tiles: [128-column block][k-chunk][16-row block][column j][half][lane] of four rows each, the
+// accumulators' own layout: lane l's unit j is rows 4 (l >> 4) .. + 3 of column
+// 64 half + 16 ((l & 15) >> 2) + (l & 3) + quarter_col(j).
+__device__ __forceinline__ size_t gemm_partial_unit(int hb, int kc, int n_kc, int rb, int n_rb, int j, int cg) {
+    return ((((size_t)hb * n_kc + kc) * n_rb + rb) * 4 + j) * GEMV_NCG + cg;
+}
+
+template <int BITS, int CB, int RB>
+__global__ __launch_bounds__(WAVE * GEMM_NKG) void gemm_kernel(
+    const u32x4_t* __restrict__ xd, const int16_t* __restrict__ trellis, int Rp, int K, int N, int nsteps, int n_kc,
+    int n_rt, int xcd, float4_t* __restrict__ partials) {
+    // the other k-groups' sums of each accumulator unit (rb, j): [unit][source][lane]
+    extern __shared__ __align__(16) char gemm_smem[];
+    float4_t* red = reinterpret_cast<float4_t*>(gemm_smem);
+    int hb, jj;
+    xcd_split(blockIdx.x, GEMV_NCG * n_kc * n_rt, xcd, hb, jj);
+    const int cg = jj & (GEMV_NCG - 1), jr = jj / GEMV_NCG;
+    const int kc = jr / n_rt, rt = jr - kc * n_rt;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int kg = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    const int g = lane >> 4, c = lane & 15, p = c & 3, n16 = N / 16;
+    const int s0 = kc * nsteps, ns = min(nsteps, K / STEP_K - s0);
+    const int row0 = rt * 16 * RB;
+
+    gptr_t<uint32_t> tp = as_global(reinterpret_cast<const uint32_t*>(trellis)) +
+                          ((size_t)(4 * (s0 + kg) + g) * n16 + 8 * hb + 4 * cg + (c >> 2)) * (8 * BITS);
+    const size_t tstep = (size_t)4 * GEMM_NKG * n16 * (8 * BITS);
+    // A unit ((s * 4 + g) * 4 + r) * Rp + row, through a buffer resource of the
+    // rotated input's size: past the wave's last step the offset lies beyond
+    // it, so the prefetch reads nothing and the loop needs no branch around it
+    const uint32_t abytes = (uint32_t)((size_t)K / STEP_K * 16 * Rp * 16);
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4_t*>(xd), (short)0, (int)abytes, 0x00020000);
+    uint32_t av = (uint32_t)((((s0 + kg) * 16 + 4 * g) * Rp + row0 + c) * 16);
+    const uint32_t astep = (uint32_t)(16 * GEMM_NKG * Rp * 16);
+
+    float4_t acc[RB][4];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[rb][q] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    QuarterTile<BITS> t0, t1;
+    half8_t A[4][RB];
+    auto load_a = [&](int r) {
+        const uint32_t v = av + (uint32_t)(r * Rp * 16);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+            A[r][rb] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(ar, v + 256 * rb, 0, 0));
+    };
+    // One step; the next step's A is requested k-group by k-group as this step's is used up.
+    auto step = [&](const QuarterTile<BITS>& t, bool more) {
+        av = more ? av + astep : 0x80000000u;
+        static_for<4>([&](auto RI) {
+            constexpr int r = decltype(RI)::value;
+            static_for<4>([&](auto JI) {
+                constexpr int q = decltype(JI)::value, n = quarter_col(q);
+                constexpr int T0 = 32 * (n & 7) + 8 * r + 4 * (n >> 3);
+                u32x4_t b;
+                b[0] = decode_pair<BITS, CB, T0 + 0>(t.w);
+                b[1] = decode_pair<BITS, CB, T0 + 1>(t.w);
+                b[2] = decode_pair<BITS, CB, T0 + 2>(t.w);
+                b[3] = decode_pair<BITS, CB, T0 + 3>(t.w);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+                    acc[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[r][rb], __builtin_bit_cast(half8_t, b),
+                                                                        acc[rb][q], 0, 0, 0);
+            });
+            __builtin_amdgcn_sched_barrier(0);         // the loads stay behind the MFMAs that read their registers
+            load_a(r);
+        });
+    };
+    if (kg < ns) {
+        load_quarter<BITS>(t0, tp, p);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) load_a(r);
+        for (int s = kg; s < ns; s += GEMM_NKG) {
+            const bool more = s + GEMM_NKG < ns;
+            tp += more ? tstep : 0;                    // past the end the last tile again
+            load_quarter<BITS>(t1, tp, p);
+            step(t0, more);
+            t0 = t1;
+        }
+    }
+
+    // Unit (rb, j) is finished by k-group j + 4 (rb & 1); the others hand it their sums.
+    static_for<4>([&](auto JI) {
+        constexpr int j = decltype(JI)::value;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const int own = j + 4 * (rb & 1);
+            if (kg != own)
+                red[((rb * 4 + j) * (GEMM_NKG - 1) + (kg < own ? kg : kg - 1)) * WAVE + lane] = acc[rb][j];
+        }
+    });
+    __syncthreads();
+    static_for<4>([&](auto JI) {
+        constexpr int j = decltype(JI)::value;
+        if ((kg & 3) == j) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                if ((rb & 1) != kg / 4) continue;
+                const float4_t* s = red + (rb * 4 + j) * (GEMM_NKG - 1) * WAVE + lane;
+                float4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < GEMM_NKG; ++k)             // k-group order
+                    v += k == kg ? acc[rb][j] : s[(k < kg ? k : k - 1) * WAVE];
+                partials[gemm_partial_unit(hb, kc, n_kc, rt * RB + rb, n_rt * RB, j, cg) * WAVE + lane] = v;
+            }
+        }
+    });
+}
+
+// Two consecutive outputs at any 2-byte alignment.
+__device__ __forceinline__ void store_out2(void* out, size_t idx, int kind, float a, float b) {
+    if (kind == OUT_F32) {
+        reinterpret_cast<float*>(out)[idx] = a;
+        reinterpret_cast<float*>(out)[idx + 1] = b;
+    } else {
+        typedef uint32_t __attribute__((aligned(2))) u32_u;
+        const uint32_t lo = kind == OUT_F16 ? f32_to_f16_bits(a) : f32_to_bf16_rne(a);
+        const uint32_t hi = kind == OUT_F16 ? f32_to_f16_bits(b) : f32_to_bf16_rne(b);
+        *reinterpret_cast<u32_u*>(reinterpret_cast<uint16_t*>(out) + idx) = lo | (hi << 16);
+    }
+}
+
+// Finish of (128-column block, 16-row block): the k-chunks' partial tiles
+// summed in chunk order, output Hadamard, svh, store.  Wave cg holds columns
+// 64 cg .. 64 cg + 63 in the accumulators' layout: stages h = 1, 2, 16, 32 run
+// between lanes (DPP), 4 and 8 in registers, 64 when the rows are read back
+// from LDS in storing order.
+template <int DUMMY = 0>
+__global__ __launch_bounds__(2 * WAVE) void gemm_finish_kernel(const float4_t* __restrict__ partials,
+                                                               const uint16_t* __restrict__ svh,
+                                                               void* __restrict__ out, int out_kind, int R, int N,
+                                                               int n_kc, int n_rb, int xcd) {
+    __shared__ float buf[MAX_ROWS * GEMV_RED_LD];
+    int hb, rb;
+    xcd_split(blockIdx.x, (R + 15) / 16, xcd, hb, rb);
+    const int lane = threadIdx.x & (WAVE - 1), cg = threadIdx.x / WAVE;
+    const int g = lane >> 4, c = lane & 15, p = c & 3;
+    float4_t v[4];
+    {
+        const float4_t* s = partials + gemm_partial_unit(hb, 0, n_kc, rb, n_rb, 0, cg) * WAVE + lane;
+        const size_t kstride = (size_t)n_rb * 4 * GEMV_NCG * WAVE;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+        constexpr int BATCH = 4;
+        for (int k0 = 0; k0 < n_kc; k0 += BATCH) {
+            float4_t t[BATCH][4];
+#pragma unroll
+            for (int k = 0; k < BATCH; ++k)
+                if (k0 + k < n_kc)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) t[k][j] = s[(k0 + k) * kstride + j * GEMV_NCG * WAVE];
+#pragma unroll
+            for (int k = 0; k < BATCH; ++k)
+                if (k0 + k < n_kc)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] += t[k][j];
+        }
+    }
+    const float s1 = (c & 1) ? -1.f : 1.f, s2 = (c & 2) ? -1.f : 1.f;
+    const float s4 = (c & 4) ? -1.f : 1.f, s8 = (c & 8) ? -1.f : 1.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][i] = bfly(v[j][i], dpp_xor<1>(v[j][i]), s1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][i] = bfly(v[j][i], dpp_xor<2>(v[j][i]), s2);
+    // units 0..3 are columns p + 0, 8, 4, 12: h = 4 pairs (0, 2), (1, 3), h = 8 pairs (0, 1), (2, 3)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const float4_t a = v[j], b = v[j + 2];
+        v[j] = a + b;
+        v[j + 2] = a - b;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+        const float4_t a = v[j], b = v[j + 1];
+        v[j] = a + b;
+        v[j + 1] = a - b;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][i] = bfly(v[j][i], dpp_xor<4>(v[j][i]), s4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][i] = bfly(v[j][i], dpp_xor<8>(v[j][i]), s8);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float* d = buf + (4 * g + i) * GEMV_RED_LD + 64 * cg + 16 * (c >> 2) + p;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[quarter_col(j)] = v[j][i];
+    }
+    __syncthreads();
+    // a half-wave per row: lane l of it columns 2l, 2l + 1 and 64 + 2l, 65 + 2l
+    const int l = lane & 31, col = 128 * hb + 2 * l;
+    float w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = f16_bits_to_f32(svh[col + (q & 1) + 64 * (q >> 1)]);
+#pragma unroll
+    for (int m0 = 0; m0 < MAX_ROWS; m0 += 4) {
+        const int m = m0 + 2 * cg + (lane >> 5), row = 16 * rb + m;
+        if (row < R) {
+            const float2 a = *reinterpret_cast<const float2*>(buf + m * GEMV_RED_LD + 2 * l);
+            const float2 b = *reinterpret_cast<const float2*>(buf + m * GEMV_RED_LD + 64 + 2 * l);
+            store_out2(out, (size_t)row * N + col, out_kind, (a.x + b.x) * HAD_NORM * w[0], (a.y + b.y) * HAD_NORM * w[1]);
+            store_out2(out, (size_t)row * N + col + 64, out_kind, (a.x - b.x) * HAD_NORM * w[2],
+                       (a.y - b.y) * HAD_NORM * w[3]);
+        }
+    }
 }
 
 // ---------------------------------------------------------------- same-input fan
@@ -675,7 +986,7 @@ constexpr int MAX_FAN = 8;
 
 struct FanParams {
     const uint16_t* x;
-    int R, K, nsteps, n_kc, count, out_kind;
+    int R, K, nsteps, n_kc, nkg, count, out_kind;
     const int16_t* trellis[MAX_FAN];
     const uint16_t* suh[MAX_FAN];
     const uint16_t* svh[MAX_FAN];
@@ -684,49 +995,35 @@ struct FanParams {
     int N[MAX_FAN];
     int bits[MAX_FAN];
     int xcd;                    // items and finish keyed by the fan's column block (xcd_split)
-    int block0[MAX_FAN + 1];    // partial-sum items: member j owns [block0[j], block0[j+1])
-    int rblock0[MAX_FAN + 1];   // finish items (128 columns x row): member j owns [rblock0[j], rblock0[j+1])
+    int hb0[MAX_FAN + 1];       // 128-column blocks: member j owns [hb0[j], hb0[j+1])
 };
 
-__device__ __forceinline__ int fan_member(const int (&first)[MAX_FAN + 1], int count, int blk) {
+__device__ __forceinline__ int fan_member(const FanParams& P, int hb) {
     int j = 0;
-    while (j + 1 < count && blk >= first[j + 1]) ++j;
+    while (j + 1 < P.count && hb >= P.hb0[j + 1]) ++j;
     return j;
 }
 
 // Items of the members with bit width BITS; the other members' items return
 // at once (one launch per width present).
-template <int BITS, int CB, int W, int RB>
-__global__ __launch_bounds__(64 * W) void gemv_fan_kernel(FanParams P) {
-    __shared__ uint16_t xa[MAX_ROWS * RB * GEMV_NSTEP_CAP * STEP_K];
+template <int BITS, int CB, int RB>
+__global__ __launch_bounds__(WAVE * GEMV_NCG * GEMV_MAX_NKG) void gemv_fan_kernel(FanParams P) {
+    extern __shared__ __align__(16) char gemv_smem[];
     // the members' column blocks in order are the fan's column blocks
-    int g, jj;
-    xcd_split(blockIdx.x, P.n_kc, P.xcd, g, jj);
-    const int i = g * P.n_kc + jj;
-    const int j = fan_member(P.block0, P.count, i);
+    int hb, kc;
+    xcd_split(blockIdx.x, P.n_kc, P.xcd, hb, kc);
+    const int j = fan_member(P, hb);
     if (P.bits[j] != BITS) return;
-    const int local = i - P.block0[j];
-    const int cb = local / P.n_kc, kc = local - (local / P.n_kc) * P.n_kc;
-    gemv_item<BITS, CB, W, RB, false>(P.x, P.trellis[j], P.suh[j], P.R, P.K, P.N[j], P.nsteps, cb, kc, P.partials[j], xa);
+    gemv_item<BITS, CB, RB>(P.x, P.trellis[j], P.suh[j], P.svh[j], P.out[j], P.out_kind, P.R, P.K, P.N[j], P.nsteps,
+                            P.n_kc, hb - P.hb0[j], kc, P.partials[j], gemv_smem);
 }
 
 template <int BATCH>
 __global__ __launch_bounds__(64) void gemv_fan_reduce_kernel(FanParams P) {
-    int g, jj;
-    xcd_split(blockIdx.x, 2 * P.R, P.xcd, g, jj);
-    const int i = g * 2 * P.R + jj;
-    const int j = fan_member(P.rblock0, P.count, i);
-    const int local = i - P.rblock0[j];
-    const int hb = local / P.R, m = local - (local / P.R) * P.R;
-    gemv_reduce_block<BATCH>(P.partials[j], P.svh[j], P.out[j], P.out_kind, P.R, P.N[j], P.n_kc, hb, m);
-}
-
-// k-chunking of a fan: as gemv_plan, over the column blocks of every member;
-// always finished by the reduction launch.
-inline GemvPlan gemv_fan_plan(int64_t rows, int64_t k, int64_t total_cb, int cus) {
-    GemvPlan p = gemv_plan_cb(rows, k, total_cb, cus);
-    p.split_reduce = true;
-    return p;
+    int hb, m;
+    xcd_split(blockIdx.x, P.R, P.xcd, hb, m);
+    const int j = fan_member(P, hb);
+    gemv_reduce_block<BATCH>(P.partials[j], P.svh[j], P.out[j], P.out_kind, P.R, P.N[j], P.n_kc, hb - P.hb0[j], m);
 }
 
 // ---------------------------------------------------------------- per-bit-width launchers
@@ -739,12 +1036,18 @@ struct DequantArgs {
 struct GemvArgs {
     const uint16_t* x; const int16_t* trellis; const uint16_t* suh; const uint16_t* svh;
     void* out; int out_kind; int R, K, N; GemvPlan plan; int codebook;
-    int* counters; float* partials; hipStream_t stream;
+    float* partials; hipStream_t stream;
+};
+
+struct GemmArgs {
+    const u32x4_t* xd; const int16_t* trellis; int K, N; GemmPlan plan; int codebook; float4_t* partials; bool xcd;
+    hipStream_t stream;
 };
 
 // Defined in exl3_dense_inst.hip, one translation unit per BITS.
 template <int BITS> int launch_dequant(const DequantArgs& a);
 template <int BITS> int launch_gemv(const GemvArgs& a);
-template <int BITS> int launch_gemv_fan(const FanParams& P, int codebook, int waves, int blocks, hipStream_t stream);
+template <int BITS> int launch_gemm(const GemmArgs& a);
+template <int BITS> int launch_gemv_fan(const FanParams& P, int codebook, hipStream_t stream);
 
 }  // namespace exl3

@@ -38,32 +38,22 @@ int launch_dequant<EXL3_BITS>(const DequantArgs& a) {
     return check_launch();
 }
 
-template <int B, int C, int W, int RB>
-static void launch_gemv_w(const GemvArgs& a) {
-    const dim3 grid(a.plan.n_cb * a.plan.n_kc), block(64 * W);
-    if (a.plan.split_reduce)
-        hipLaunchKernelGGL((gemv_kernel<B, C, W, RB, true>), grid, block, 0, a.stream, a.x, a.trellis, a.suh,
-                           a.svh, a.out, a.out_kind, a.R, a.K, a.N, a.plan.nsteps, a.plan.n_kc, a.plan.xcd ? 1 : 0,
-                           a.counters, a.partials);
-    else
-        hipLaunchKernelGGL((gemv_kernel<B, C, W, RB, false>), grid, block, 0, a.stream, a.x, a.trellis, a.suh,
-                           a.svh, a.out, a.out_kind, a.R, a.K, a.N, a.plan.nsteps, a.plan.n_kc, a.plan.xcd ? 1 : 0,
-                           a.counters, a.partials);
-}
-
-// Up to 16 rows: one MFMA row block, 1, 2 or 4 column groups; 17-32 rows:
-// two row blocks, 2 or 4 column groups (the plan never picks 1 there).
+// Up to 16 rows: one MFMA row block; 17-32 rows: two.
 template <>
 int launch_gemv<EXL3_BITS>(const GemvArgs& a) {
     constexpr int B = EXL3_BITS;
+    const GemvPlan& p = a.plan;
+    const dim3 grid(p.n_hb * p.n_kc), block(WAVE * GEMV_NCG * p.nkg);
+    const int lds = gemv_lds_bytes(a.R, p.nsteps, p.nkg);
     auto go = [&](auto cbc) {
         constexpr int C = decltype(cbc)::value;
-        if (a.R > MAX_ROWS) {
-            if (a.plan.waves == 4) launch_gemv_w<B, C, 4, 2>(a);
-            else launch_gemv_w<B, C, 2, 2>(a);
-        } else if (a.plan.waves == 4) launch_gemv_w<B, C, 4, 1>(a);
-        else if (a.plan.waves == 2) launch_gemv_w<B, C, 2, 1>(a);
-        else launch_gemv_w<B, C, 1, 1>(a);
+        auto launch = [&](auto rbc) {
+            hipLaunchKernelGGL((gemv_kernel<B, C, decltype(rbc)::value>), grid, block, lds, a.stream, a.x, a.trellis,
+                               a.suh, a.svh, a.out, a.out_kind, a.R, a.K, a.N, p.nsteps, p.n_kc, p.xcd ? 1 : 0,
+                               a.partials);
+        };
+        if (a.R > MAX_ROWS) launch(std::integral_constant<int, 2>{});
+        else launch(std::integral_constant<int, 1>{});
     };
     switch (a.codebook) {
         case CB_MCG: go(std::integral_constant<int, CB_MCG>{}); break;
@@ -74,17 +64,42 @@ int launch_gemv<EXL3_BITS>(const GemvArgs& a) {
 }
 
 template <>
-int launch_gemv_fan<EXL3_BITS>(const FanParams& P, int codebook, int waves, int blocks, hipStream_t stream) {
+int launch_gemm<EXL3_BITS>(const GemmArgs& a) {
     constexpr int B = EXL3_BITS;
+    const GemmPlan& p = a.plan;
+    const dim3 grid(p.n_hb * GEMV_NCG * p.n_kc * p.n_rt), block(WAVE * GEMM_NKG);
     auto go = [&](auto cbc) {
         constexpr int C = decltype(cbc)::value;
-        const dim3 grid(blocks);
-        if (P.R > MAX_ROWS) {
-            if (waves == 4) hipLaunchKernelGGL((gemv_fan_kernel<B, C, 4, 2>), grid, dim3(256), 0, stream, P);
-            else hipLaunchKernelGGL((gemv_fan_kernel<B, C, 2, 2>), grid, dim3(128), 0, stream, P);
-        } else if (waves == 4) hipLaunchKernelGGL((gemv_fan_kernel<B, C, 4, 1>), grid, dim3(256), 0, stream, P);
-        else if (waves == 2) hipLaunchKernelGGL((gemv_fan_kernel<B, C, 2, 1>), grid, dim3(128), 0, stream, P);
-        else hipLaunchKernelGGL((gemv_fan_kernel<B, C, 1, 1>), grid, dim3(64), 0, stream, P);
+        auto launch = [&](auto rbc) {
+            constexpr int RB = decltype(rbc)::value;
+            constexpr int lds = 4 * RB * (GEMM_NKG - 1) * WAVE * (int)sizeof(float4_t);
+            hipLaunchKernelGGL((gemm_kernel<B, C, RB>), grid, block, lds, a.stream, a.xd, a.trellis, p.n_rt * 16 * p.rb,
+                               a.K, a.N, p.nsteps, p.n_kc, p.n_rt, a.xcd ? 1 : 0, a.partials);
+        };
+        switch (p.rb) {
+            case 2: launch(std::integral_constant<int, 2>{}); break;
+            case 3: launch(std::integral_constant<int, 3>{}); break;
+            case 4: launch(std::integral_constant<int, 4>{}); break;
+            default: launch(std::integral_constant<int, 5>{}); break;
+        }
+    };
+    switch (a.codebook) {
+        case CB_MCG: go(std::integral_constant<int, CB_MCG>{}); break;
+        case CB_3INST: go(std::integral_constant<int, CB_3INST>{}); break;
+        default: go(std::integral_constant<int, CB_MUL1>{}); break;
+    }
+    return check_launch();
+}
+
+template <>
+int launch_gemv_fan<EXL3_BITS>(const FanParams& P, int codebook, hipStream_t stream) {
+    constexpr int B = EXL3_BITS;
+    const dim3 grid(P.hb0[P.count] * P.n_kc), block(WAVE * GEMV_NCG * P.nkg);
+    const int lds = gemv_lds_bytes(P.R, P.nsteps, P.nkg);
+    auto go = [&](auto cbc) {
+        constexpr int C = decltype(cbc)::value;
+        if (P.R > MAX_ROWS) hipLaunchKernelGGL((gemv_fan_kernel<B, C, 2>), grid, block, lds, stream, P);
+        else hipLaunchKernelGGL((gemv_fan_kernel<B, C, 1>), grid, block, lds, stream, P);
     };
     switch (codebook) {
         case CB_MCG: go(std::integral_constant<int, CB_MCG>{}); break;

@@ -116,8 +116,8 @@ __device__ __forceinline__ uint16_t decode_half(const uint32_t* W) {
 // item of group g runs on XCD g % 8, and so does the reader's item for g.
 // Item j of group g is workgroup 8 (per_group (g / 8) + j) + g % 8, a
 // bijection onto the same grid when the group count is a multiple of 8.
-// The dense GEMV and its split-K finish use it (16 rows of 4096x4096: 14.0
-// against 16.0 us); in the routed-MoE phased launches the same keys (gate/up
+// The dense kernels and their split-K finish use it (16 rows of 4096x4096 with
+// 256-column items of 128 k-rows: 14.0 against 16.0 us); in the routed-MoE phased launches the same keys (gate/up
 // by column block of I, down and finish by column block of H) measured the
 // same as the slot-major order at 1-16 rows, so they keep that order.
 constexpr int N_XCD = 8;
@@ -440,6 +440,31 @@ __device__ __forceinline__ void fwht128_x8(float (&v)[8]) {
     for (int e = 0; e < 8; ++e) v[e] = bfly(v[e], dpp_xor<8>(v[e]), s8);
 }
 
+// half(x * s) of 8 packed inputs (fp16 or bf16 x, fp16 s), as fp32.
+__device__ __forceinline__ void scaled8(const u32x4_t& xv, const u32x4_t& sv, int x_kind, float (&v)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint16_t xb = (uint16_t)(h ? xv[i] >> 16 : xv[i] & 0xffffu);
+            const uint16_t x16 = x_kind != 0 ? f32_to_f16_bits(bf16_to_f32(xb)) : xb;
+            const uint16_t s16 = (uint16_t)(h ? sv[i] >> 16 : sv[i] & 0xffffu);
+            // the fp32 product of two halves is exact, so one RNE cast = half mul
+            v[2 * i + h] = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(x16) * f16_bits_to_f32(s16)));
+        }
+    }
+}
+
+// The block transform of 8 values per lane, normalised and rounded to fp16.
+__device__ __forceinline__ u32x4_t rotated8(float (&v)[8]) {
+    fwht128_x8(v);
+    u32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        o[i] = (uint32_t)f32_to_f16_bits(v[2 * i] * HAD_NORM) | ((uint32_t)f32_to_f16_bits(v[2 * i + 1] * HAD_NORM) << 16);
+    return o;
+}
+
 // Same transform for two independent 128-blocks, 4 consecutive elements per
 // lane: lanes 0-31 hold block 0, lanes 32-63 block 1 (element 4j+e of the block
 // in lane j of the half-wave).
@@ -489,18 +514,6 @@ __device__ __forceinline__ void had_in_load(const void* x, size_t x_off, const u
             in.x[b] = xp[64 * b];
             in.s[b] = sp[64 * b];
         }
-}
-
-// The lane's two rotated elements (2l, 2l+1) of one 128-block, packed as fp16
-// in natural order, from its loaded input pair v2 (x_kind) and sign pair s2.
-__device__ __forceinline__ uint32_t had_in_pair(uint32_t v2, uint32_t s2, int x_kind) {
-    if (x_kind != 0)
-        v2 = (uint32_t)f32_to_f16_bits(bf16_to_f32((uint16_t)(v2 & 0xffffu))) |
-             ((uint32_t)f32_to_f16_bits(bf16_to_f32((uint16_t)(v2 >> 16))) << 16);
-    float v0 = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(v2 & 0xffffu) * f16_bits_to_f32(s2 & 0xffffu)));
-    float v1 = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(v2 >> 16) * f16_bits_to_f32(s2 >> 16)));
-    fwht128_x2(v0, v1);
-    return (uint32_t)f32_to_f16_bits(v0 * HAD_NORM) | ((uint32_t)f32_to_f16_bits(v1 * HAD_NORM) << 16);
 }
 
 __device__ __forceinline__ void had_in_store(const RowIn& in, int x_kind, uint16_t* xa, int m, int nblocks,

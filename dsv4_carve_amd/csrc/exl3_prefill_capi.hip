@@ -164,30 +164,6 @@ __global__ __launch_bounds__(1024) void pf_plan_kernel(PfParams P) {
 // columns, so the chain of dependent loads (pair -> scale pointers -> x and
 // scales) is paid once for both.
 
-// half(x * s) of 8 packed inputs (fp16 or bf16 x, fp16 s), as fp32.
-__device__ __forceinline__ void pf_scaled8(const u32x4_t& xv, const u32x4_t& sv, int x_kind, float (&v)[8]) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint16_t xb = (uint16_t)(h ? xv[i] >> 16 : xv[i] & 0xffffu);
-            const uint16_t x16 = x_kind != 0 ? f32_to_f16_bits(bf16_to_f32(xb)) : xb;
-            const uint16_t s16 = (uint16_t)(h ? sv[i] >> 16 : sv[i] & 0xffffu);
-            // the fp32 product of two halves is exact, so one RNE cast = half mul
-            v[2 * i + h] = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(x16) * f16_bits_to_f32(s16)));
-        }
-    }
-}
-
-__device__ __forceinline__ u32x4_t pf_rotated8(float (&v)[8]) {
-    fwht128_x8(v);
-    u32x4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        o[i] = (uint32_t)f32_to_f16_bits(v[2 * i] * HAD_NORM) | ((uint32_t)f32_to_f16_bits(v[2 * i + 1] * HAD_NORM) << 16);
-    return o;
-}
-
 __global__ __launch_bounds__(64) void pf_rotate_kernel(PfParams P) {
     const PfLayout& L = P.L;
     const int nch = (P.H + 511) / 512;
@@ -205,9 +181,9 @@ __global__ __launch_bounds__(64) void pf_rotate_kernel(PfParams P) {
     const u32x4_t gs = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(P.gsu[e]) + cl);
     const u32x4_t us = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint16_t*>(P.usu[e]) + cl);
     float vg[8], vu[8];
-    pf_scaled8(xv, gs, P.x_kind, vg);
-    pf_scaled8(xv, us, P.x_kind, vu);
-    const u32x4_t og = pf_rotated8(vg), ou = pf_rotated8(vu);
+    scaled8(xv, gs, P.x_kind, vg);
+    scaled8(xv, us, P.x_kind, vu);
+    const u32x4_t og = rotated8(vg), ou = rotated8(vu);
     uint16_t* xh = pat<uint16_t>(P.scratch, L.Xh);
     if (live) {
         *reinterpret_cast<u32x4_t*>(xh + (size_t)p * P.H + col) = og;

@@ -17,6 +17,7 @@ Reference call surfaces mirrored here:
 
 from __future__ import annotations
 
+import functools
 import threading
 
 import torch
@@ -307,16 +308,29 @@ def had_r_128(x: torch.Tensor, y: torch.Tensor, pre_scale: torch.Tensor | None, 
     torch.ops.exl3_amd.had_rows(x, y, pre_scale, post_scale, float(scale))
 
 
+GEMV_MAX_ROWS = 32
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_scratch_bytes(device_index: int, m: int, k: int, n: int) -> int:
+    return int(_lib.check(_lib.load().exl3_gemm_scratch_bytes(m, k, n)))
+
+
 def gemm_scratch(device: torch.device, m: int, k: int, n: int) -> torch.Tensor:
-    nbytes = _lib.check(_lib.load().exl3_gemm_scratch_bytes(m, k, n))
+    """Scratch of a dense call: the shared buffer up to 32 rows (reserved before a graph capture by
+    prepare_gemm), the call's own temporary above (stream-ordered, and a capture may allocate it)."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    nbytes = _gemm_scratch_bytes(int(index), int(m), int(k), int(n))
+    if m > GEMV_MAX_ROWS:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
     return SCRATCH.get(device, "gemm", nbytes)
 
 
 def prepare_gemm(device: torch.device, max_rows: int, k: int, n: int) -> None:
     """Reserve the shared dense scratch before any graph capture (the role of
-    LNA_EXL3_PREWARM_ROWS, recipe-lna/vllm_exl3_exl3.py.lna:2718-2742)."""
-    for m in range(1, max_rows + 1):
-        gemm_scratch(device, m, k, n)
+    LNA_EXL3_PREWARM_ROWS, recipe-lna/vllm_exl3_exl3.py.lna:2718-2742).  The size
+    for a row count serves every smaller one."""
+    gemm_scratch(device, min(int(max_rows), GEMV_MAX_ROWS), k, n)
 
 
 def gemm_into(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,

@@ -6,10 +6,10 @@ error behaviour, so the plugin's dispatch code can switch to this package:
   * ``LinearEXL3`` / ``make_linear_exl3`` / ``execute_exl3_linear`` -- the
     exllamav3 linear (recipe-lna/exllamav3/exl3.py.lna:16-218,
     recipe-lna/vllm_exl3_exl3.py.lna:889-926).  Up to AUTO_RECONSTRUCT_THRESHOLD
-    rows run the trellis-decode GEMV kernel; more rows reconstruct the fp16
-    weight on the GPU and run one hgemm, between row-Hadamard launches below
-    FUSED_RECONSTRUCT_MIN_ROWS rows and on the Hadamard-folded weight from
-    there on.
+    rows run the trellis-decode GEMV kernel, up to GEMM_MAX_ROWS its many-row
+    form; more rows reconstruct the fp16 weight on the GPU and run one hgemm,
+    between row-Hadamard launches below FUSED_RECONSTRUCT_MIN_ROWS rows and on
+    the Hadamard-folded weight from there on.
   * ``apply_exl3_experts`` and its helpers -- routed experts
     (recipe-lna/vllm_exl3_exl3.py.lna:951-1296, 1543-1569, 1707-1779): backend
     selection by VLLM_EXL3_MOE_KERNEL, strict levels by VLLM_EXL3_MOE_STRICT,
@@ -58,15 +58,17 @@ MUL1_MULTIPLIER = 0x83DCD12D
 MUL1_MARKER_SIGNED_INT32 = -2082680531
 EXL3_SUFFIXES = ("trellis", "suh", "svh", "mcg", "mul1")
 SWIGLU_LIMIT_DEFAULT = 10.0
-# Rows up to AUTO_RECONSTRUCT_THRESHOLD take the decode GEMV; more take the
-# reconstruct path.  The reference switches at 144 rows
-# (recipe-lna/exllamav3/exl3.py.lna:10); on MI355X the GEMV is faster up to 32
-# rows (one 32-row block) and the reconstruct path from 48 rows on the
-# 4096x4096, 4096x1536, 1536x4096 and 4096x12288 matrices (at 144 rows the
-# GEMV takes 2.8x its time on 4096x4096).  From FUSED_RECONSTRUCT_MIN_ROWS
-# rows the rotations are folded into the reconstructed weight (the
-# reference's rule, exl3.py.lna:184).
+# Rows up to AUTO_RECONSTRUCT_THRESHOLD take the decode GEMV (shared scratch,
+# reserved before capture), more the decode GEMM up to GEMM_MAX_ROWS, and the
+# reconstruct path above.  The reference switches at 144 rows
+# (recipe-lna/exllamav3/exl3.py.lna:10).  On MI355X, us per call, GEMM /
+# reconstruct: 4096x4096 4-bit 256 rows 34 / 40, 384 rows 48 / 44; 4096x12288
+# 6-bit 256 rows 73 / 89, 512 rows 149 / 106; 1536x4096 256 rows 20 / 29, 512
+# rows 38 / 35; 8192x8192 256 rows 81 / 116, 384 rows 125 / 110.  From
+# FUSED_RECONSTRUCT_MIN_ROWS rows the rotations are folded into the
+# reconstructed weight (the reference's rule, exl3.py.lna:184).
 AUTO_RECONSTRUCT_THRESHOLD = 32
+GEMM_MAX_ROWS = 256
 FUSED_RECONSTRUCT_MIN_ROWS = 1024
 MAX_RECONSTRUCT_SLICE_N = 32768
 MOE_TABLE_KEYS = ops.MOE_TABLE_KEYS
@@ -148,7 +150,7 @@ class LinearEXL3:
         assert x.is_contiguous(), f"LinearEXL3 {self.key}: non-contiguous input {tuple(x.shape)}"
         dtype = out_dtype or self.default_out_dtype
         rows = x.numel() // x.shape[-1]
-        if not params.get("reconstruct") and (rows <= AUTO_RECONSTRUCT_THRESHOLD
+        if not params.get("reconstruct") and (rows <= GEMM_MAX_ROWS
                                               or self.config.infer_params.no_reconstruct):
             x2 = x.view(rows, self.in_features)
             if x2.dtype != torch.float16:
@@ -402,14 +404,15 @@ def _dense_prewarm_rows() -> tuple[int, ...]:
 
 
 def _prewarm_group(group: dict, outs_for=None) -> bool:
-    """Runs the fused call once per prewarm row count (and at the largest row
-    count the group runs, so every later row count fits) so the shared scratch
-    exists before any capture.  False (logged) on failure."""
+    """Runs the fused call once per prewarm row count (the largest row count the
+    group runs first, so the scratch is allocated once and every later row count
+    fits) so the shared scratch exists before any capture.  False (logged) on
+    failure."""
     device = group["device"]
     if device.type != "cuda":
         return False
     try:
-        for rows in sorted(set(_dense_prewarm_rows()) | {DENSE_GROUP_MAX_ROWS}):
+        for rows in sorted(set(_dense_prewarm_rows()) | {DENSE_GROUP_MAX_ROWS}, reverse=True):
             x = torch.zeros((rows, group["k"]), dtype=torch.float16, device=device)
             ops.gemm_group(x, group["members"], group["codebook"], torch.float32,
                            outs=None if outs_for is None else outs_for(rows))

@@ -68,10 +68,10 @@ int exl3_had_rows(const void* x, int x_kind, void* y, int y_kind, int64_t rows, 
  * limits k % 16, n % 128 at :35-37) as used by LinearEXL3.forward for rows <= 144
  * (recipe-lna/exllamav3/exl3.py.lna:114-139), and vllm_exl3_c.exl3_gemv
  * (recipe-lna/lna2/bindings.cpp:135-148).  a: fp16 [m][k]; k % 128 == 0,
- * n % 128 == 0; any m (processed in blocks of 16 rows).  scratch: device
- * buffer of at least exl3_gemm_scratch_bytes(m, k, n) bytes, zeroed once
- * before its first use; the kernels leave its counters zero again, so one
- * buffer serves every later call on the same stream (one call at a time).
+ * n % 128 == 0; any m (in blocks of 32 rows, or 256 on the many-row kernels).
+ * scratch: device buffer of at least exl3_gemm_scratch_bytes(m, k, n) bytes
+ * (which serves every call of up to m rows; no zeroing needed); one call at a
+ * time per scratch buffer.
  */
 int64_t exl3_gemm_scratch_bytes(int64_t m, int64_t k, int64_t n);
 int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t n, int bits,

@@ -308,3 +308,79 @@ def test_xcd_keyed_order_is_bitwise_the_plain_order(ops, dev, monkeypatch, rows)
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     ref = O.linear(x_np, L["trellis"], L["suh"], L["svh"], bits, O.CB_MCG)
     assert_close(keyed[0], ref, what=f"keyed order rows={rows}")
+
+
+@pytest.mark.parametrize("k,n,bits,rows", [
+    (128, 128, 3, 1),         # the smallest: 2 steps, one workgroup, finished in its launch
+    (384, 128, 6, 16),        # 6 steps in chunks of 4: a short last chunk
+    (2176, 256, 2, 5),        # 34 steps: a last chunk of 2 steps for 4 k-groups
+    (640, 384, 5, 17),        # two row blocks, an odd column-block count
+    (4096, 128, 1, 32),       # one column block, every k-chunk on it
+    (256, 8192, 3, 20),       # 17-32 rows on many columns: the many-row kernels
+    (128, 128, 4, 33),        # fewer steps than k-groups
+    (896, 256, 8, 80),        # a whole row tile of 5 row blocks, 14 steps
+    (1152, 384, 7, 81),       # one row more: two row tiles of 3 row blocks
+    (4096, 256, 6, 160),      # two whole row tiles
+    (512, 128, 3, 256),       # a whole slab
+    (512, 256, 2, 257),       # one row more: a second slab of one row
+])
+def test_gemm_tile_edges(ops, dev, k, n, bits, rows):
+    """Edges of the dense kernels' tiles and splits, against the oracle on the
+    weights they use (each weight's exact addend sum): fp32 sums of k products
+    in any order, so sqrt(k) 2^-24 <= 4e-6 relative at these k; measured below
+    4e-7, asserted at 2e-6."""
+    import torch
+
+    got, ref = _gemm_case(ops, dev, k, n, bits, rows, torch.float32, seed=500 + k + n + rows)
+    assert_close(got, ref, what=f"{k}x{n} K{bits} rows={rows}")
+    L = synth.dense(k, n, bits, seed=500 + k + n + rows + bits)
+    x = synth.activations(rows, k, seed=500 + k + n + 2 * rows)
+    exact = O.linear(x, L["trellis"], L["suh"], L["svh"], bits, O.CB_MCG,
+                     w=O.reconstruct_exact(L["trellis"], bits, O.CB_MCG))
+    assert_close(got, exact, max_abs=2e-5, rel=2e-6, what=f"{k}x{n} K{bits} rows={rows} (exact addends)")
+
+
+@pytest.mark.parametrize("rows", [3, 20, 70])
+def test_gemm_unaligned_operands(ops, dev, rows):
+    """x, suh, svh and the output at odd half-element addresses (contiguous
+    views into larger buffers) give bitwise the aligned call's output."""
+    import torch
+
+    k, n, bits = 512, 256, 3
+    L = synth.dense(k, n, bits, seed=41)
+    t, u, v = (to_dev(L[key], dev) for key in ("trellis", "suh", "svh"))
+    x = to_dev(synth.activations(rows, k, seed=42), dev)
+
+    def odd(a):
+        buf = torch.empty(a.numel() + 1, dtype=a.dtype, device=dev)
+        buf[1:] = a.reshape(-1)
+        return buf[1:].view(a.shape)
+
+    for dt in (torch.float16, torch.bfloat16, torch.float32):
+        want = ops.gemm(x, t, u, v, ops.CB_MCG, dt)
+        got = ops.gemm_into(odd(x), t, odd(u), odd(v), odd(torch.empty_like(want)), ops.CB_MCG)
+        assert torch.equal(got, want), dt
+
+
+def test_many_row_linear_captures_without_prewarm(dev):
+    """A linear of more than 32 rows captured with no earlier call (its scratch
+    is the call's own) replays bitwise what the eager call gives, with other
+    eager calls and a synchronize between the replays."""
+    import torch
+
+    from dsv4_carve_amd import vllm_exl3 as V
+
+    L = synth.dense(1024, 512, 4, seed=51)
+    mcg = torch.tensor([V.MCG_MARKER_SIGNED_INT32], dtype=torch.int32, device=dev)
+    lin = V.make_linear_exl3(*(to_dev(L[key], dev) for key in ("trellis", "suh", "svh")), mcg)
+    x = to_dev(synth.activations(72, 1024, seed=52), dev)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = lin.forward(x, {}, out_dtype=torch.float32)
+    for seed in (53, 54, 55):
+        x.copy_(to_dev(synth.activations(72, 1024, seed=seed), dev))
+        want = lin.forward(x, {}, out_dtype=torch.float32)
+        lin.forward(torch.randn(40, 1024, device=dev).half(), {})
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
