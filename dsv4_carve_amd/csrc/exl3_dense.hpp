@@ -66,43 +66,65 @@ __global__ __launch_bounds__(64) void dequant_raw_kernel(const int16_t* __restri
     }
 }
 
+// 8 consecutive halves at any 2-byte alignment, as one 16-byte load where the
+// target allows it.
+__device__ __forceinline__ u32x4_t load_half8(const uint16_t* p) {
+    typedef u32x4_t __attribute__((aligned(2))) u32x4_u;
+    return *(gptr_t<u32x4_u>)p;
+}
+
 // ---------------------------------------------------------------- dequant (Hadamard folded)
 
 // W = diag(suh) H Wq H diag(svh) / 128 in the operation order of dequant_cpu
 // (recipe-lna/lna2/bindings.cpp:80-99): row transforms (* 1/sqrt(128)), then
-// column transforms, value = ((v*norm)*su)*sv.  One workgroup of four waves
+// column transforms, value = ((v*norm)*su)*sv.  One workgroup of eight waves
 // per 128x128 block:
-//   1. rows: lane l of every wave owns tile (l >> 3, l & 7) of the block and
-//      wave w its tile rows 4w..4w+3.  A tile row's 16 values are decoded into
-//      registers, transformed by butterflies h = 1..8 in registers and
-//      h = 16, 32, 64 with the lanes of the same tile row (lane ^ 1, 2, 4),
-//      normalised, and written to LDS as fp32.
-//   2. columns: wave w owns columns 32w..32w+31, lanes l and l ^ 32 the upper
-//      and lower 64 rows of column 32w + (l & 31): butterflies h = 1..32 in
-//      registers, h = 64 across the two lanes, then norm, su, sv, fp16.
+//   1. rows: a lane owns one tile of the block and wave w its tile rows 2w and
+//      2w + 1.  A tile row's 16 values are decoded into registers, transformed
+//      by butterflies h = 1..8 in registers and h = 16, 32, 64 with the lanes of
+//      the same tile row (lane ^ 1, 2, 8: one DPP move each), normalised, and
+//      written to LDS as fp32.
+//   2. columns: wave w owns columns 16w..16w+15, the lanes of 16-lane row q the
+//      rows 32q..32q+31 of them: butterflies h = 1..16 in registers; for h = 32
+//      and 64 two registers swap 16- and 32-lane rows, which brings both
+//      operands of two butterflies into one lane; then norm, su, sv, fp16.
 // The butterfly stages run in the order h = 1, 2, ..., 64 of the reference's
 // scalar loop and every butterfly is a single fp32 add or subtract of the same
 // two operands, so the result is bitwise the loop's.
 //
+// Bound by its ~30 VALU instructions per weight, so by waves in flight: the fp32
+// block is 64 KB of LDS, two workgroups a CU, and eight waves each make four a
+// SIMD.  Against four waves a workgroup, with the last column stage through the
+// LDS permute and whole tiles decoded by 16-bit multiplies: 4096x4096 at 3 bits
+// 28.2 -> 19.1 us ([n][k]), 25.0 -> 19.5 ([k][n]); 4096x12288 at 6 bits 70.1 ->
+// 51.6 and 62.2 -> 52.2.
+//
 // LDS position of block element (r, c), fp32, unpadded: 16-byte chunks are
-// XOR-swizzled within each aligned group of 8 by the tile column (c >> 4) & 7,
-// so the eight lanes of a tile row writing the same chunk of their own tiles,
-// and 32 lanes reading 32 consecutive columns of one row, fall on distinct
-// banks.
+// XOR-swizzled by the tile column (c >> 4) & 7, so the lanes of a tile row
+// writing the same chunk of their own tiles fall on distinct banks, and by r >> 5,
+// so the four 16-lane rows reading 16 columns of rows 32 apart do.
 __device__ __forceinline__ int hb_pos(int r, int c) {
-    return r * 128 + ((((c >> 2) ^ ((c >> 4) & 7)) << 2) | (c & 3));
+    return r * 128 + ((((c >> 2) ^ ((c >> 4) & 7) ^ (((r >> 5) & 3) << 2)) << 2) | (c & 3));
 }
 
-// Phase 1 for tile rows K0..K0+3 of this lane's tile.
+// The value of lane ^ 8 of a 16-lane row (rotation by half a row).
+__device__ __forceinline__ float dpp_ror8(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xF, 0xF, false));
+}
+
+// Phase 1 for tile rows K0, K0 + 1 of this lane's tile (kt, nt).  s1, s2, s4:
+// -1 in the lanes whose nt has that bit, else 1.
 template <int BITS, int CB, int K0>
-__device__ __forceinline__ void had_rows(const uint32_t* W, int kt, int nt, float* mat) {
-    const float s1 = (nt & 1) ? -1.f : 1.f, s2 = (nt & 2) ? -1.f : 1.f, s4 = (nt & 4) ? -1.f : 1.f;
-    static_for<4>([&](auto KI) {
+__device__ __forceinline__ void had_rows(const uint32_t* W, int kt, int nt, float s1, float s2, float s4, float* mat) {
+    static_for<2>([&](auto KI) {
         constexpr int k = K0 + decltype(KI)::value;
         float v[16];
         static_for<16>([&](auto NI) {
             constexpr int n = decltype(NI)::value;
-            v[n] = f16_bits_to_f32(decode_half<BITS, CB, tile_t(k, n)>(W));
+            const uint32_t x = decode_pair<BITS, CB, tile_t(k, n)>(W);
+            const _Float16 lo = __builtin_bit_cast(_Float16, (uint16_t)x);
+            if constexpr (CB == CB_MUL1) v[n] = (float)lo;
+            else v[n] = (float)(_Float16)(lo + __builtin_bit_cast(_Float16, (uint16_t)(x >> 16)));
         });
 #pragma unroll
         for (int h = 1; h < 16; h <<= 1)
@@ -118,7 +140,7 @@ __device__ __forceinline__ void had_rows(const uint32_t* W, int kt, int nt, floa
 #pragma unroll
         for (int n = 0; n < 16; ++n) v[n] = bfly(v[n], dpp_xor<2>(v[n]), s2);
 #pragma unroll
-        for (int n = 0; n < 16; ++n) v[n] = bfly(v[n], dpp_xor<4>(v[n]), s4);
+        for (int n = 0; n < 16; ++n) v[n] = bfly(v[n], dpp_ror8(v[n]), s4);
         const int r = 16 * kt + k;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -128,84 +150,110 @@ __device__ __forceinline__ void had_rows(const uint32_t* W, int kt, int nt, floa
     });
 }
 
+// Butterfly across 16-lane rows 2i, 2i + 1 (ROWS 16) or 32-lane halves (ROWS 32)
+// of two registers: after the swap a lane of an even row (lower half) holds both
+// operands of a's butterfly, one of an odd row (upper half) those of b's.  a
+// becomes their sum, b the lower minus the upper.
+template <int ROWS>
+__device__ __forceinline__ void swap_bfly(float& a, float& b) {
+    unsigned lo, hi;
+    if constexpr (ROWS == 16) {
+        const auto t = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                        false, false);
+        lo = t[0];
+        hi = t[1];
+    } else {
+        const auto t = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b),
+                                                        false, false);
+        lo = t[0];
+        hi = t[1];
+    }
+    const float x = __builtin_bit_cast(float, lo), y = __builtin_bit_cast(float, hi);
+    a = x + y;
+    b = x - y;
+}
+
 template <int BITS, int CB, bool NK = false>
-__global__ __launch_bounds__(256) void dequant_had_kernel(const int16_t* __restrict__ trellis, int k16,
-                                                          int n16, const uint16_t* __restrict__ suh,
-                                                          const uint16_t* __restrict__ svh,
-                                                          uint16_t* __restrict__ out) {
+__global__ __launch_bounds__(512, 4) void dequant_had_kernel(const int16_t* __restrict__ trellis, int k16,
+                                                             int n16, const uint16_t* __restrict__ suh,
+                                                             const uint16_t* __restrict__ svh,
+                                                             uint16_t* __restrict__ out) {
     __shared__ __align__(16) float mat[128 * 128];
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     const int nbc = n16 / 8;
     const int br = blockIdx.x / nbc, bc = blockIdx.x - br * nbc;
     const size_t N = (size_t)n16 * 16;
     {
-        const int kt = lane >> 3, nt = lane & 7;
+        const int nt = (lane & 3) | ((lane >> 1) & 4), kt = ((lane >> 2) & 1) | ((lane >> 3) & 6);
+        const float s1 = (nt & 1) ? -1.f : 1.f, s2 = (nt & 2) ? -1.f : 1.f, s4 = (nt & 4) ? -1.f : 1.f;
         TileRegs<BITS> t;
         load_tile<BITS>(t, reinterpret_cast<const u32x4_t*>(trellis) +
                                ((size_t)(8 * br + kt) * n16 + 8 * bc + nt) * tile_vecs<BITS>());
         const uint32_t* W = t.words();
         switch (wave) {
-            case 0: had_rows<BITS, CB, 0>(W, kt, nt, mat); break;
-            case 1: had_rows<BITS, CB, 4>(W, kt, nt, mat); break;
-            case 2: had_rows<BITS, CB, 8>(W, kt, nt, mat); break;
-            default: had_rows<BITS, CB, 12>(W, kt, nt, mat); break;
+            case 0: had_rows<BITS, CB, 0>(W, kt, nt, s1, s2, s4, mat); break;
+            case 1: had_rows<BITS, CB, 2>(W, kt, nt, s1, s2, s4, mat); break;
+            case 2: had_rows<BITS, CB, 4>(W, kt, nt, s1, s2, s4, mat); break;
+            case 3: had_rows<BITS, CB, 6>(W, kt, nt, s1, s2, s4, mat); break;
+            case 4: had_rows<BITS, CB, 8>(W, kt, nt, s1, s2, s4, mat); break;
+            case 5: had_rows<BITS, CB, 10>(W, kt, nt, s1, s2, s4, mat); break;
+            case 6: had_rows<BITS, CB, 12>(W, kt, nt, s1, s2, s4, mat); break;
+            default: had_rows<BITS, CB, 14>(W, kt, nt, s1, s2, s4, mat); break;
         }
     }
-    const int c = 32 * wave + (lane & 31), half = lane >> 5;
-    // this lane's 64 row scales (128 contiguous bytes), requested before the barrier
-    u32x4_t su4[8];
-    const u32x4_t* sp = reinterpret_cast<const u32x4_t*>(suh + 128 * br + 64 * half);
+    const int c = 16 * wave + (lane & 15), q = lane >> 4;
+    // after the swaps this lane's rows are k0 + 32 i + j, i < 4, j < 8
+    const int k0 = 16 * (q & 1) + 8 * (q >> 1);
+    u32x4_t su4[4];                                // requested before the barrier
 #pragma unroll
-    for (int i = 0; i < 8; ++i) su4[i] = sp[i];
+    for (int i = 0; i < 4; ++i) su4[i] = load_half8(suh + 128 * br + k0 + 32 * i);
     const float sv = f16_bits_to_f32(svh[128 * bc + c]);
     __syncthreads();
-    float v[64];
+    float v[32];
 #pragma unroll
-    for (int j = 0; j < 64; ++j) v[j] = mat[hb_pos(64 * half + j, c)];
-    __syncthreads();                               // mat is free: it becomes the fp16 output tile
+    for (int j = 0; j < 32; ++j) v[j] = mat[hb_pos(32 * q + j, c)];
+    if constexpr (!NK) __syncthreads();            // mat is free: it becomes the fp16 output tile
 #pragma unroll
-    for (int h = 1; h < 64; h <<= 1)
+    for (int h = 1; h < 32; h <<= 1)
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
+        for (int j = 0; j < 16; ++j) {
             const int i = (j / h) * 2 * h + (j % h);
             const float a = v[i], b = v[i + h];
             v[i] = a + b;
             v[i + h] = a - b;
         }
-    const uint32_t* su = reinterpret_cast<const uint32_t*>(su4);
-    const float s32 = half ? -1.f : 1.f;
-    if constexpr (NK) {
-        // this lane's 64 values are consecutive along k in output row n = 128 bc + c
-        uint32_t pk[32];
+    // h = 32: v[j], j < 16, becomes row 64 (q >> 1) + 16 (q & 1) + j, v[j + 16] the row 32 below
 #pragma unroll
-        for (int j = 0; j < 64; ++j) {
-            float x = bfly(v[j], shfl_xor(v[j], 32), s32);
-            x = x * HAD_NORM;
-            x = x * f16_bits_to_f32((uint16_t)(su[j >> 1] >> (16 * (j & 1))));
-            x = x * sv;
-            const uint32_t h = f32_to_f16_bits(x);
-            pk[j >> 1] = (j & 1) ? (pk[j >> 1] | (h << 16)) : h;
-        }
-        const size_t K = (size_t)k16 * 16;
-        u32x4_t* o = reinterpret_cast<u32x4_t*>(out + (size_t)(128 * bc + c) * K + 128 * br + 64 * half);
+    for (int j = 0; j < 16; ++j) swap_bfly<16>(v[j], v[j + 16]);
+    // h = 64: of the first 16, v[j], j < 8, becomes row k0 + j and v[j + 8] row 64 + k0 + j; the second 32 below
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = u32x4_t{pk[4 * i], pk[4 * i + 1], pk[4 * i + 2], pk[4 * i + 3]};
-        return;
-    }
+    for (int j = 0; j < 8; ++j) swap_bfly<32>(v[j], v[j + 8]);
+#pragma unroll
+    for (int j = 16; j < 24; ++j) swap_bfly<32>(v[j], v[j + 8]);
     uint16_t* o16 = reinterpret_cast<uint16_t*>(mat);
 #pragma unroll
-    for (int j = 0; j < 64; ++j) {
-        float x = bfly(v[j], shfl_xor(v[j], 32), s32);
-        x = x * HAD_NORM;
-        x = x * f16_bits_to_f32((uint16_t)(su[j >> 1] >> (16 * (j & 1))));
-        x = x * sv;
-        o16[(64 * half + j) * 128 + c] = f32_to_f16_bits(x);
+    for (int i = 0; i < 4; ++i) {
+        // rows k0 + 32 i ..: i = 0, 1, 2, 3 in v[0..7], v[16..23], v[8..15], v[24..31]
+        const int b = 16 * (i & 1) + 8 * (i >> 1);
+        u32x4_t o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            float x = v[b + j] * HAD_NORM;
+            x = x * f16_bits_to_f32((uint16_t)(su4[i][j >> 1] >> (16 * (j & 1))));
+            x = x * sv;
+            const uint32_t h = f32_to_f16_bits(x);
+            if constexpr (NK) o[j >> 1] = (j & 1) ? (o[j >> 1] | (h << 16)) : h;
+            else o16[(k0 + 32 * i + j) * 128 + c] = (uint16_t)h;
+        }
+        if constexpr (NK)
+            *reinterpret_cast<u32x4_t*>(out + (size_t)(128 * bc + c) * ((size_t)k16 * 16) + 128 * br + k0 + 32 * i) = o;
     }
+    if constexpr (NK) return;
     __syncthreads();
     // 128 rows x 256 bytes, 16 bytes per lane and pass
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int id = i * 256 + (int)threadIdx.x, row = id >> 4, seg = id & 15;
+    for (int i = 0; i < 4; ++i) {
+        const int id = i * 512 + (int)threadIdx.x, row = id >> 4, seg = id & 15;
         *reinterpret_cast<u32x4_t*>(out + (size_t)(128 * br + row) * N + 128 * bc + 8 * seg) =
             *reinterpret_cast<const u32x4_t*>(o16 + row * 128 + 8 * seg);
     }
@@ -395,13 +443,6 @@ inline int64_t gemv_partial_bytes(int64_t rows, int64_t n_hb, int64_t n_kc) {
 }
 __device__ __forceinline__ size_t gemv_partial_off(int hb, int row, int kc, int R, int n_kc) {
     return ((size_t)(hb * R + row) * n_kc + kc) * GEMV_COLS;
-}
-
-// 8 consecutive halves at any 2-byte alignment, as one 16-byte load where the
-// target allows it.
-__device__ __forceinline__ u32x4_t load_half8(const uint16_t* p) {
-    typedef u32x4_t __attribute__((aligned(2))) u32x4_u;
-    return *(gptr_t<u32x4_u>)p;
 }
 
 // The words of a lane's quarter tile: rotated blocks 0 and 4 and the word

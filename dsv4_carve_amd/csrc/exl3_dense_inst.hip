@@ -15,10 +15,10 @@ int launch_dequant<EXL3_BITS>(const DequantArgs& a) {
         if (a.suh) {
             const int blocks = (a.k16 / 8) * (a.n16 / 8);
             if (a.nk)
-                hipLaunchKernelGGL((dequant_had_kernel<B, C, true>), dim3(blocks), dim3(256), 0, a.stream, a.trellis,
+                hipLaunchKernelGGL((dequant_had_kernel<B, C, true>), dim3(blocks), dim3(512), 0, a.stream, a.trellis,
                                    a.k16, a.n16, a.suh, a.svh, a.out);
             else
-                hipLaunchKernelGGL((dequant_had_kernel<B, C, false>), dim3(blocks), dim3(256), 0, a.stream,
+                hipLaunchKernelGGL((dequant_had_kernel<B, C, false>), dim3(blocks), dim3(512), 0, a.stream,
                                    a.trellis, a.k16, a.n16, a.suh, a.svh, a.out);
         } else {
             const int tiles = a.k16 * a.n16;
