@@ -392,15 +392,67 @@ __device__ __forceinline__ float bfly(float own, float partner, float sgn) {
 }
 
 
+// The butterfly of lanes l and l ^ M (M a power of two below 64): the sum in the
+// lane without bit M, partner minus own in the other; sgn is 1 and -1 there.
+// Without LDS traffic: by DPP within 16 lanes, beyond by swapping 16- or 32-lane
+// rows of two copies, which leaves the lower lane's value in one and the upper's
+// in the other.  A shuffle through the LDS permute is ~120 cycles a stage, and a
+// 128-point transform is a chain of five or six of them in every item's
+// prologue and finish.  With the shuffles, input
+// rotated at 4.5 us and down input ready at 7.5 us of a 1-row launch of the
+// 256-expert layer; now 4.3 and 7.2, and the finish kernels are ~0.5 us shorter.
+template <int M>
+__device__ __forceinline__ float xlane_bfly(float v, float sgn) {
+    if constexpr (M <= 8) {
+        return bfly(v, dpp_xor<M>(v), sgn);
+    } else {
+        const unsigned u = __builtin_bit_cast(unsigned, v);
+        unsigned lo, hi;
+        if constexpr (M == 16) {
+            const auto t = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+            lo = t[0];
+            hi = t[1];
+        } else {
+            static_assert(M == 32, "below 64");
+            const auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+            lo = t[0];
+            hi = t[1];
+        }
+        return bfly(__builtin_bit_cast(float, hi), __builtin_bit_cast(float, lo), sgn);
+    }
+}
+
+// Stages M = 1, 2, 4, ... below LANES of N elements per lane.
+template <int LANES, int M = 1, int N>
+__device__ __forceinline__ void xlane_stages(float (&v)[N]) {
+    if constexpr (M < LANES) {
+        const float sgn = (threadIdx.x & M) ? -1.f : 1.f;
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = xlane_bfly<M>(v[e], sgn);
+        xlane_stages<LANES, 2 * M>(v);
+    }
+}
+
 // In-place natural-order 128-point FWHT of a block held as 2 consecutive
 // elements per lane (element 2l+e in lane l), fp32, same add/sub sequence per
 // element as the scalar loop in orders/F1-ref/exl3_dequant.cuh:136-147.
+// SWAP false: shuffles through the LDS permute (bitwise the same).  The ticket
+// MoE kernel keeps them: its all-width instance sits at 256 registers and would
+// spill 58 values instead of 50.
+template <bool SWAP = true>
 __device__ __forceinline__ void fwht128_x2(float& v0, float& v1) {
     const int lane = threadIdx.x & (WAVE - 1);
     {
         const float a = v0, b = v1;
         v0 = a + b;
         v1 = a - b;
+    }
+    if constexpr (SWAP) {
+        float v[2] = {v0, v1};
+        xlane_stages<64>(v);
+        v0 = v[0];
+        v1 = v[1];
+        return;
     }
 #pragma unroll
     for (int m = 1; m < 64; m <<= 1) {
@@ -468,6 +520,7 @@ __device__ __forceinline__ u32x4_t rotated8(float (&v)[8]) {
 // Same transform for two independent 128-blocks, 4 consecutive elements per
 // lane: lanes 0-31 hold block 0, lanes 32-63 block 1 (element 4j+e of the block
 // in lane j of the half-wave).
+template <bool SWAP = true>
 __device__ __forceinline__ void fwht128_x4(float (&v)[4]) {
     const int lane = threadIdx.x & (WAVE - 1);
     {
@@ -479,6 +532,10 @@ __device__ __forceinline__ void fwht128_x4(float (&v)[4]) {
         v[0] = a + b; v[2] = a - b;
         a = v[1]; b = v[3];
         v[1] = a + b; v[3] = a - b;
+    }
+    if constexpr (SWAP) {
+        xlane_stages<32>(v);
+        return;
     }
 #pragma unroll
     for (int m = 1; m < 32; m <<= 1) {
@@ -516,6 +573,7 @@ __device__ __forceinline__ void had_in_load(const void* x, size_t x_off, const u
         }
 }
 
+template <bool SWAP = true>
 __device__ __forceinline__ void had_in_store(const RowIn& in, int x_kind, uint16_t* xa, int m, int nblocks,
                                              int nsteps_cap) {
     const int lane = threadIdx.x & (WAVE - 1);
@@ -529,18 +587,19 @@ __device__ __forceinline__ void had_in_store(const RowIn& in, int x_kind, uint16
         // half(x*suh): the fp32 product of two halves is exact, so one RNE cast = half mul
         float v0 = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(v2 & 0xffffu) * f16_bits_to_f32(in.s[b] & 0xffffu)));
         float v1 = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(v2 >> 16) * f16_bits_to_f32(in.s[b] >> 16)));
-        fwht128_x2(v0, v1);
+        fwht128_x2<SWAP>(v0, v1);
         const int k0 = 128 * b + 2 * lane;
         xa[xa_index(m, k0 >> 6, nsteps_cap, k0 & 63)] = f32_to_f16_bits(v0 * HAD_NORM);
         xa[xa_index(m, (k0 + 1) >> 6, nsteps_cap, (k0 + 1) & 63)] = f32_to_f16_bits(v1 * HAD_NORM);
     }
 }
 
+template <bool SWAP = true>
 __device__ __forceinline__ void had_in_row(const void* x, size_t x_off, int x_kind, const uint16_t* suh,
                                            uint16_t* xa, int m, int nblocks, int nsteps_cap) {
     RowIn in;
     had_in_load(x, x_off, suh, nblocks, in);
-    had_in_store(in, x_kind, xa, m, nblocks, nsteps_cap);
+    had_in_store<SWAP>(in, x_kind, xa, m, nblocks, nsteps_cap);
 }
 
 // Input rotation of the rows in `mask` (row r of the tile = the r-th set bit)
@@ -548,7 +607,7 @@ __device__ __forceinline__ void had_in_row(const void* x, size_t x_off, int x_ki
 // inputs are requested before the tile, the rest after it.
 constexpr int IN_AHEAD = 2;
 
-template <int BITS>
+template <int BITS, bool SWAP = true>
 __device__ __forceinline__ void rotate_rows_and_load(const void* x, size_t row_stride, size_t k0, int x_kind,
                                                      const uint16_t* suh, uint32_t mask, uint16_t* xa, int nblocks,
                                                      int nsteps_cap, TileRegs<BITS>& first, const u32x4_t* tp) {
@@ -565,11 +624,11 @@ __device__ __forceinline__ void rotate_rows_and_load(const void* x, size_t row_s
     load_tile<BITS>(first, tp);
 #pragma unroll
     for (int i = 0; i < IN_AHEAD; ++i)
-        if (i < R) had_in_store(in[i], x_kind, xa, i, nblocks, nsteps_cap);
+        if (i < R) had_in_store<SWAP>(in[i], x_kind, xa, i, nblocks, nsteps_cap);
     for (int r = IN_AHEAD; r < R; ++r) {
         const int row = __ffs((int)rest) - 1;
         rest &= rest - 1u;
-        had_in_row(x, (size_t)row * row_stride + k0, x_kind, suh, xa, r, nblocks, nsteps_cap);
+        had_in_row<SWAP>(x, (size_t)row * row_stride + k0, x_kind, suh, xa, r, nblocks, nsteps_cap);
     }
 }
 
