@@ -840,6 +840,47 @@ __device__ __forceinline__ bool slot_group(const Params& P, int o, SlotGroup& g,
     return true;
 }
 
+// Down input of one (row, 128-block) unit: pair `pair` at intermediate columns
+// [k0, k0 + 128), into row 0 of the LDS A tile.  The lower half-wave sums and
+// rotates the gate column block, the upper the up one, each with all its chunk
+// loads in flight (up to 32), then a row swap gives both halves both values.
+// For calls of one row with chunks of one block, where down_input_chunk would
+// leave a half-wave idle and double the chain (256-expert layer 45.3 -> 44.6 us,
+// TP slice 23.3 -> 22.2).  With more units both half-waves have one of their own
+// and splitting each loses (16 rows on hot experts of 32: 44 -> 59 us), and both
+// forms in one kernel cost its other items 1-2%, so it is an instance of its own.
+__device__ __forceinline__ void down_input_unit(const Params& P, int e, int pair, uint16_t* xa, int k0) {
+    const Layout& L = P.L;
+    const int lane = threadIdx.x & (WAVE - 1), half = lane >> 5;
+    const int kk = 4 * (lane & 31), col = k0 + kk;
+    uint16_t sv[4], dsu[4];
+    load_half4(sv, (half ? P.usv : P.gsv)[e], col);
+    load_half4(dsu, P.dsu[e], col);
+    const uint32_t cb = (uint32_t)col / COLS, c = (uint32_t)col % COLS;
+    const float4_t t = sum_partials<CPOL_PLAIN>(
+        at<float>(P.scratch, L.PA),
+        (((uint32_t)pair * 2u + (uint32_t)half) * (uint32_t)(L.SA * P.I) + cb * (uint32_t)(L.SA * COLS) + c) * 4u, COLS,
+        L.SA);
+    float v[4] = {t[0], t[1], t[2], t[3]};
+    fwht128_x4(v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const unsigned w = __builtin_bit_cast(unsigned, v[i] * HAD_NORM * f16_bits_to_f32(sv[i]));
+        const auto gu = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+        const unsigned gg = gu[0], uu = gu[1];
+        const uint16_t act =
+            f32_to_f16_bits(silu_clamped(__builtin_bit_cast(float, gg), __builtin_bit_cast(float, uu), P.limit));
+        // down input rotation: half(act * down_suh), fp32 butterflies
+        v[i] = f16_bits_to_f32(f32_to_f16_bits(f16_bits_to_f32(act) * f16_bits_to_f32(dsu[i])));
+    }
+    fwht128_x4(v);
+    // both halves hold the row: each stores two of its four values
+    const float a = half ? v[2] : v[0], b = half ? v[3] : v[1];
+    const int k2 = kk + 2 * half;
+    xa[xa_index(0, k2 >> 6, NSTEP_CAP, k2 & 63)] = f32_to_f16_bits(a * HAD_NORM);
+    xa[xa_index(0, (k2 + 1) >> 6, NSTEP_CAP, (k2 + 1) & 63)] = f32_to_f16_bits(b * HAD_NORM);
+}
+
 // Down input of the rows pslot[0..R) at intermediate columns [k0, k0 + kchunk)
 // (kchunk a multiple of 128), written into the LDS A tile: each half-wave
 // computes one (row, 128-block) unit per pass (its butterflies never leave the
@@ -939,7 +980,8 @@ __global__ __launch_bounds__(64) void moe_slot_act(Params P) {
 // batches (fuse_act) the item first computes its chunk of the down input (the
 // activation of the gate/up sums) into LDS while its first weight tile is in
 // flight; otherwise it copies that chunk from the activation launch's DI.
-template <uint32_t MASK, int CB>
+// ONE_UNIT: one row and chunks of 128, fuse_act (down_input_unit).
+template <uint32_t MASK, int CB, bool ONE_UNIT>
 __global__ __launch_bounds__(64, 2) void moe_slot_down(Params P) {
     extern __shared__ __align__(16) uint16_t xa[];   // moe_lds_kb(m, E) KB
     __shared__ int16_t pslot[MAX_M];
@@ -968,7 +1010,10 @@ __global__ __launch_bounds__(64, 2) void moe_slot_down(Params P) {
                 const u32x4_t* tp = tile_ptr<B>(reinterpret_cast<const int16_t*>(P.dt[g.e]), P.H / 16,
                                                 kc * kchunk / 16, cb * 16);
                 TileRegs<B> first;
-                if (P.fuse_act) {
+                if constexpr (ONE_UNIT) {
+                    load_tile<B>(first, tp);
+                    down_input_unit(P, g.e, ps[0], xa, kc * kchunk);
+                } else if (P.fuse_act) {
                     load_tile<B>(first, tp);
                     down_input_chunk(P, g.e, R, ps, xa, kc * kchunk, kchunk);
                 } else {

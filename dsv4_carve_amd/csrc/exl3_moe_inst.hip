@@ -33,8 +33,11 @@ int launch_phased<EXL3_MOE_MASK, EXL3_MOE_CB>(const Params& P, int lds_kb, hipSt
         hipLaunchKernelGGL((moe_slot_act<0>), dim3(slots * L.nI), dim3(WAVE), 0, stream, P);
         if ((rc = check_launch())) return rc;
     }
-    hipLaunchKernelGGL((moe_slot_down<EXL3_MOE_MASK, EXL3_MOE_CB>), dim3(slots * L.nH * L.SB), dim3(WAVE), lds,
-                       stream, P);
+    const dim3 grid(slots * L.nH * L.SB);
+    if (P.m == 1 && P.fuse_act && L.stepsB * STEP_K == 128)
+        hipLaunchKernelGGL((moe_slot_down<EXL3_MOE_MASK, EXL3_MOE_CB, true>), grid, dim3(WAVE), lds, stream, P);
+    else
+        hipLaunchKernelGGL((moe_slot_down<EXL3_MOE_MASK, EXL3_MOE_CB, false>), grid, dim3(WAVE), lds, stream, P);
     if ((rc = check_launch())) return rc;
     hipLaunchKernelGGL((moe_slot_finish<0>), dim3(L.nH * P.m), dim3(P.topk * WAVE), 0, stream, P);
     return check_launch();
