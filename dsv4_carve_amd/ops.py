@@ -88,11 +88,29 @@ class _ScratchPool:
                         torch.cuda.synchronize(buf.device)
                     del self._bufs[key]
                     del buf
-                buf = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
+                buf = self._allocate(max(nbytes, 256), device)
                 self._bufs[key] = buf
             if capturing:
                 self._captured.add(key)
             return buf
+
+    @staticmethod
+    def _allocate(nbytes: int, device: torch.device) -> torch.Tensor:
+        """A zeroed buffer in a block of its own size.
+
+        The allocator hands out a cached block whole where less than 1 MiB of
+        it would be left over, and a buffer of this pool would keep that excess
+        for the process's life.  Such a block is set aside while another is
+        asked for (a few times at most; a buffer of more than 32 MiB takes what
+        it gets)."""
+        aside = []
+        while device.type == "cuda" and nbytes <= 32 << 20 and len(aside) < 8:
+            before = torch.cuda.memory_allocated(device)
+            buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            if torch.cuda.memory_allocated(device) - before < nbytes + 512:
+                return buf.zero_()
+            aside.append(buf)
+        return torch.zeros(nbytes, dtype=torch.uint8, device=device)
 
     def current(self, device: torch.device, purpose: str) -> torch.Tensor | None:
         idx = device.index if device.index is not None else torch.cuda.current_device()

@@ -220,3 +220,21 @@ def test_vram_trace_phases_match_the_scratch_sizes(dev, monkeypatch, caplog):
     assert delta["registration.local_tables"] == 0.0
     assert near("registration.local_scratch", blocks(held["gemm_group"]))
     assert near("first_call", 2 * blocks(m * I * 4))
+
+
+@pytest.mark.parametrize("mib", [2.0, 2.25])
+def test_scratch_takes_no_oversized_cached_block(mib):
+    """A scratch buffer beside a 3 MiB hole of the allocator's cache, which is
+    too small to be split, is given a block of its own size."""
+    import torch
+
+    from dsv4_carve_amd import ops
+
+    dev = torch.device("cuda", 0)
+    held = [torch.empty(3 << 20, dtype=torch.uint8, device=dev) for _ in range(8)]
+    held[3] = None
+    nbytes = int(mib * 2 ** 20)
+    before = torch.cuda.memory_allocated(dev)
+    buf = ops.SCRATCH._allocate(nbytes, dev)
+    grown = torch.cuda.memory_allocated(dev) - before
+    assert nbytes <= grown < nbytes + 512 and int(buf.count_nonzero()) == 0
