@@ -149,8 +149,8 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
     return 0;
 }
 
-// Fan scratch: per member, its split-K partials (gemv_partial_bytes), each
-// member's region 256-byte aligned.
+// Scratch of exactly this fan call: per member, its split-K partials
+// (gemv_partial_bytes), each member's region 256-byte aligned.
 static int64_t fan_scratch(int64_t m, int64_t k, int64_t count, const int64_t* n_list, int cus, GemvPlan* plan,
                            int64_t* offsets) {
     int64_t total_hb = 0;
@@ -180,7 +180,12 @@ static int check_fan(int64_t m, int64_t k, int64_t count, const int64_t* n_list)
 int64_t exl3_gemm_group_scratch_bytes(int64_t m, int64_t k, int64_t count, const int64_t* n_list) {
     clear_error();
     if (int rc = check_fan(m, k, count, n_list)) return rc;
-    return fan_scratch(m, k, count, n_list, device_cus(), nullptr, nullptr);
+    // enough for every call of up to m rows: fewer rows may take more k-chunks
+    const int cus = device_cus();
+    int64_t most = 0;
+    for (int64_t r = 1; r <= m && r <= GEMV_MAX_ROWS; ++r)
+        most = std::max(most, fan_scratch(r, k, count, n_list, cus, nullptr, nullptr));
+    return most;
 }
 
 int exl3_gemm_group(const uint16_t* a, int64_t m, int64_t k, int64_t count, const int16_t* const* trellis,

@@ -379,11 +379,18 @@ def gemm(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.T
 MAX_GROUP = 8
 
 
-def gemm_group_scratch(device: torch.device, m: int, k: int, ns) -> torch.Tensor:
+@functools.lru_cache(maxsize=4096)
+def _gemm_group_scratch_bytes(device_index: int, m: int, k: int, ns: tuple[int, ...]) -> int:
     import ctypes
 
-    arr = (ctypes.c_int64 * len(ns))(*[int(n) for n in ns])
-    nbytes = _lib.check(_lib.load().exl3_gemm_group_scratch_bytes(m, k, len(ns), arr))
+    arr = (ctypes.c_int64 * len(ns))(*ns)
+    return int(_lib.check(_lib.load().exl3_gemm_group_scratch_bytes(m, k, len(ns), arr)))
+
+
+def gemm_group_scratch(device: torch.device, m: int, k: int, ns) -> torch.Tensor:
+    """The shared buffer of the fused calls.  The size for a row count serves every smaller one."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    nbytes = _gemm_group_scratch_bytes(int(index), int(m), int(k), tuple(int(n) for n in ns))
     return SCRATCH.get(device, "gemm_group", nbytes)
 
 

@@ -88,8 +88,9 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
  * bit width and need not be ordered widest first.  trellis/suh/svh/c: host
  * arrays of count device pointers; n_list: host int64 [count], each a multiple
  * of 128; bits_list: host int32 [count] in 1..8; every c_j has c_kind.
- * scratch: >= exl3_gemm_group_scratch_bytes(m, k, count, n_list) bytes (no
- * zeroing needed); one call at a time per scratch buffer.
+ * scratch: >= exl3_gemm_group_scratch_bytes(m, k, count, n_list) bytes (which
+ * serves every call of up to m rows; no zeroing needed); one call at a time per
+ * scratch buffer.
  */
 int64_t exl3_gemm_group_scratch_bytes(int64_t m, int64_t k, int64_t count, const int64_t* n_list);
 int exl3_gemm_group(const uint16_t* a, int64_t m, int64_t k, int64_t count, const int16_t* const* trellis,

@@ -320,6 +320,40 @@ def test_linear_method_prewarms_groups_and_captures(dev):
     assert V.dense_group_call_counts()[1] > 0
 
 
+@pytest.mark.parametrize("k,shards,bits", [(2048, [1024, 1024], 4), (3072, [512, 512], 3)])
+def test_default_buckets_serve_captures_at_every_row_count(dev, k, shards, bits):
+    """Shapes whose fused call takes more k-chunks at 9-13 rows than at 16: the
+    default row buckets reserve enough for a capture at each of 1..16 rows, the
+    captured call is the fused one, and its replays match the eager call."""
+    import torch
+    from dsv4_carve_amd import ops, vllm_exl3 as V
+
+    V.reset_dense_group_state()
+    pool, ops.SCRATCH = ops.SCRATCH, ops._ScratchPool()      # nothing reserved by earlier tests
+    try:
+        with dense_group(1):
+            layer, meth, host = _quant_module(dev, "model.layers.3.ffn.shared_experts.gate_up_proj", k, shards,
+                                              bits, seed=1250)
+            before = ops.SCRATCH.resident_bytes()
+            for rows in range(1, 17):
+                x16 = synth.activations(rows, k, seed=1260 + rows)
+                x = to_dev(x16.astype(np.float32), dev)
+                calls = V.dense_group_call_counts()[1]
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph):
+                    static_out = meth.apply(layer, x)
+                assert V.dense_group_call_counts()[1] == calls + 1, f"rows={rows}: not the fused call"
+                want = meth.apply(layer, x).clone()
+                for rep in range(2):
+                    graph.replay()
+                    torch.cuda.synchronize()
+                    assert torch.equal(static_out, want), f"rows={rows} replay {rep}"
+                assert_close(want.cpu().numpy(), _module_ref(host, x16), what=f"rows={rows}")
+            assert ops.SCRATCH.resident_bytes() == before, "a call needed scratch the prewarm did not reserve"
+    finally:
+        ops.SCRATCH = pool
+
+
 def _attention_fans(dev, k=1024, seed=1400):
     """One attention layer's T1 members: the h-fan (fused_wqa_wkv with two
     shards, compressor and indexer compressor with two each) and the q-fan

@@ -154,6 +154,18 @@ def test_prefill_pair_limit_without_device():
     assert _routed_call("exl3_moe_prefill_routed", m=32769, topk=2) == -1 and "65536" in _err()
 
 
+def test_fan_scratch_serves_every_smaller_row_count():
+    """What is reserved at one row count is enough at every smaller one: the
+    k-chunks of a fan call depend on its rows, and fewer rows may take more
+    (2048 -> 1024 + 1024: 16 chunks at 9-13 rows, 8 at 16)."""
+    lib = _lib.load()
+    for k, ns in ((2048, (1024, 1024)), (3072, (512, 512)), (2560, (1152,)), (1024, (512, 512)),
+                  (4096, (1024, 512, 1024, 1024, 256, 256)), (1024, (32768, 8192))):
+        arr = (ctypes.c_int64 * len(ns))(*ns)
+        size = [_lib.check(lib.exl3_gemm_group_scratch_bytes(m, k, len(ns), arr)) for m in range(1, 41)]
+        assert size == sorted(size), (k, ns)
+
+
 def test_prefill_scratch_drops_where_k_stops_splitting():
     """The prefill GEMMs split K in two below 4096 (down) and 8192 (gate/up)
     (token, slot) pairs and keep it whole from there, so the scratch, which
