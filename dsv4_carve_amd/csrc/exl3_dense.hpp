@@ -369,11 +369,14 @@ struct GemvPlan {
 inline int64_t gemv_block_rows(int64_t m) { return m > MAX_ROWS ? GEMV_MAX_ROWS : MAX_ROWS; }
 
 // EXL3_GEMV_STEPS overrides the plan's steps per k-chunk (an even number; read
-// at every call).
+// once per process: the sizes callers reserve for depend on it).
 inline int gemv_steps_override() {
-    const char* v = getenv("EXL3_GEMV_STEPS");
-    const int x = v && *v ? atoi(v) : 0;
-    return x >= 2 && x % 2 == 0 ? x : 0;
+    static const int steps = [] {
+        const char* v = getenv("EXL3_GEMV_STEPS");
+        const int x = v && *v ? atoi(v) : 0;
+        return x >= 2 && x % 2 == 0 ? x : 0;
+    }();
+    return steps;
 }
 
 // Rows of the A tile in LDS, odd so that the units of neighbouring k-slices

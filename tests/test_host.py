@@ -166,6 +166,17 @@ def test_fan_scratch_serves_every_smaller_row_count():
         assert size == sorted(size), (k, ns)
 
 
+def test_chunk_override_is_read_once(monkeypatch):
+    """A change of EXL3_GEMV_STEPS after the first dense call changes no plan:
+    a size that was reserved (and is kept by the ops) stays enough."""
+    lib = _lib.load()
+    size = lambda: _lib.check(lib.exl3_gemm_scratch_bytes(1, 4096, 4096))
+    first = size()
+    for steps in ("2", "32"):
+        monkeypatch.setenv("EXL3_GEMV_STEPS", steps)
+        assert size() == first, steps
+
+
 def test_prefill_scratch_drops_where_k_stops_splitting():
     """The prefill GEMMs split K in two below 4096 (down) and 8192 (gate/up)
     (token, slot) pairs and keep it whole from there, so the scratch, which
