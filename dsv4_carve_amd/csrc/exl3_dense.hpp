@@ -325,7 +325,7 @@ __global__ __launch_bounds__(64) void had_rows_kernel(const void* x, int x_kind,
 //
 // y = had_in(x) . Wq for rows 0..R-1 (R <= 32), split over workgroups by
 // 128-column block (one output Hadamard block) and k-chunk.  A workgroup is
-// 2 x nkg waves (nkg = 2, 4 or 8): column half cg (64 columns, 4 n-tiles) and
+// 2 x nkg waves (nkg = 2, 4 or 8; gemv_plan_hb): column half cg (64 columns, 4 n-tiles) and
 // k-group kg, which takes the chunk's 64-row steps kg, kg + nkg, ...  The
 // k-groups' sums meet in LDS, so a k-chunk of 512 rows leaves one partial
 // vector, and a call whose chunk is all of K is finished in the same launch.
@@ -356,6 +356,7 @@ constexpr int GEMV_COLS = 128;      // columns per workgroup: one Hadamard block
 constexpr int GEMV_NCG = 2;         // column halves per workgroup
 constexpr int GEMV_MAX_NKG = 8;     // k-groups per workgroup
 constexpr int GEMV_MAX_ROWS = 32;   // rows per call: one or two 16-row MFMA blocks share each decode
+constexpr int GEMV_LDS = 160 << 10;  // bytes a CU has
 constexpr int GEMV_RED_LD = 130;    // row stride (floats) of the k-groups' sums in LDS
 
 struct GemvPlan {
@@ -415,10 +416,51 @@ inline GemvPlan gemv_plan_hb(int64_t rows, int64_t k, int64_t total_hb, int cus)
             nsteps = ns;
         }
     }
-    if (env_steps && env_steps <= cap) nsteps = env_steps < S ? env_steps : S;
     p.nsteps = nsteps;
-    p.n_kc = (S + nsteps - 1) / nsteps;
-    p.nkg = nsteps >= 8 ? 8 : nsteps >= 4 ? 4 : 2;
+    p.nkg = nsteps >= 8 ? GEMV_MAX_NKG : nsteps >= 4 ? 4 : 2;
+    // Eight k-groups make a workgroup that fills a CU, whose start, exchange and
+    // finish nothing covers: where a launch is several such workgroups a CU, two
+    // or four k-groups leave room for others to decode meanwhile.  Expected time
+    // (us) by k-groups and, where K is split anyway, chunk length: a launch's
+    // start, rounds of the workgroups a CU holds (by waves and by LDS), each a
+    // start and its longest chain of steps, less the more there are to cover it,
+    // and the steps' decode and rotation.  Only chunks of 8 steps and more: below
+    // that the first choice holds four waves a SIMD already.  One round is left as
+    // it is unless the gain is clear.  On 63 shapes (512x256 to 4096x129280, 1-32
+    // rows, 1-6 bits) at most 2% slower than the first choice with eight k-groups,
+    // which one-wave items of whole tiles had beaten by up to 15% there; us, those
+    // items / eight k-groups / this rule: 512x129280 2-bit 1 row 14.8 / 17.4 / 12.4;
+    // 4096x65536 2-bit 1 row 37.9 / 42.1 / 37.9; 4096x129280 6-bit 1 row 100 / 103 /
+    // 85; 8192x65536 6-bit 4 rows 105 / 113 / 96; 4096x12288 2-bit 4 rows 14.3 /
+    // 14.6 / 12.5.
+    if (nsteps >= 8) {
+        auto time = [&](int ns, int nkg) {
+            constexpr double covered[5] = {1.0, 1.0, 0.86, 0.79, 0.74};
+            const int64_t n_kc = (S + ns - 1) / ns, per_cu = (total_hb * n_kc + cus - 1) / cus;
+            const int resident = std::max(std::min(GEMV_MAX_NKG / nkg, GEMV_LDS / gemv_lds_bytes(r, ns, nkg)), 1);
+            double t = 2.4 + std::max((double)per_cu / resident, 1.0) * (1.44 + 0.4 * ns / nkg) * covered[resident];
+            t += (double)(per_cu * ns) * (0.205 * (r > MAX_ROWS ? 1.55 : 1.0) + 0.014 * (double)r);
+            if (n_kc > 1) t += 2.06 + 0.0267 * (double)n_kc + 4.6e-7 * (double)(n_kc * r * total_hb * GEMV_COLS);
+            return t;
+        };
+        const bool whole = nsteps >= S;
+        const bool rounds = total_hb * ((S + nsteps - 1) / nsteps) > cus;
+        double least = time(nsteps, GEMV_MAX_NKG) * (rounds ? 1.0 : 0.9);
+        for (int ns = whole ? S : 8; ns <= (whole ? S : std::min(cap, S - 1)); ns += 8)
+            for (int nkg = 2; nkg <= GEMV_MAX_NKG; nkg *= 2) {
+                const double t = time(ns, nkg);
+                if (t < least) {
+                    least = t;
+                    p.nsteps = ns;
+                    p.nkg = nkg;
+                }
+            }
+    }
+    if (env_steps && env_steps <= cap) {
+        p.nsteps = env_steps < S ? env_steps : S;
+        p.nkg = p.nsteps >= 8 ? GEMV_MAX_NKG : p.nsteps >= 4 ? 4 : 2;
+    }
+    p.n_kc = (S + p.nsteps - 1) / p.nsteps;
     return p;
 }
 
@@ -766,7 +808,10 @@ inline GemmPlan gemm_plan(int64_t R, int64_t k, int64_t n, int cus) {
 inline int64_t dense_scratch_bytes(int64_t rows, int64_t k, int64_t n, int cus) {
     if (!gemm_takes(rows, k, n)) {
         const GemvPlan p = gemv_plan(rows, k, n, cus);
-        return align_up(gemv_partial_bytes(rows, p.n_hb, p.n_kc), 256) + 256;
+        const int64_t b = align_up(gemv_partial_bytes(rows, p.n_hb, p.n_kc), 256) + 256;
+        return rows > GEMV_MAX_ROWS && rows % GEMV_MAX_ROWS
+                   ? std::max(b, dense_scratch_bytes(rows % GEMV_MAX_ROWS, k, n, cus))    // the last block
+                   : b;
     }
     const GemmPlan g = gemm_plan(rows < GEMM_MAX_ROWS ? rows : GEMM_MAX_ROWS, k, n, cus);
     int64_t b = align_up(g.xd_bytes, 256) + g.partial_bytes;

@@ -340,6 +340,25 @@ def test_gemm_tile_edges(ops, dev, k, n, bits, rows):
     assert_close(got, exact, max_abs=2e-5, rel=2e-6, what=f"{k}x{n} K{bits} rows={rows} (exact addends)")
 
 
+@pytest.mark.parametrize("k,n,bits,rows", [
+    (512, 33024, 2, 1),       # whole K on four k-groups, two workgroups of some CUs
+    (512, 33024, 6, 16),      # the same with a full row block
+    (640, 33152, 3, 5),       # 10 steps on four k-groups
+    (2176, 16512, 1, 5),      # chunks of 8 steps on two k-groups, the last of 2
+])
+def test_long_launch_k_groups(ops, dev, k, n, bits, rows):
+    """Launches of more workgroups than CUs, which take fewer k-groups each,
+    against the oracle on the weights they use (bound as in test_gemm_tile_edges)."""
+    import torch
+
+    got, _ = _gemm_case(ops, dev, k, n, bits, rows, torch.float32, seed=700 + rows)
+    L = synth.dense(k, n, bits, seed=700 + rows + bits)
+    x = synth.activations(rows, k, seed=700 + 2 * rows)
+    exact = O.linear(x, L["trellis"], L["suh"], L["svh"], bits, O.CB_MCG,
+                     w=O.reconstruct_exact(L["trellis"], bits, O.CB_MCG))
+    assert_close(got, exact, max_abs=2e-5, rel=2e-6, what=f"{k}x{n} K{bits} rows={rows}")
+
+
 @pytest.mark.parametrize("rows", [3, 20, 70])
 def test_gemm_unaligned_operands(ops, dev, rows):
     """x, suh, svh and the output at odd half-element addresses (contiguous
