@@ -64,7 +64,8 @@ SWIGLU_LIMIT_DEFAULT = 10.0
 # (recipe-lna/exllamav3/exl3.py.lna:10).  On MI355X, us per call, GEMM /
 # reconstruct: 4096x4096 4-bit 256 rows 34 / 40, 384 rows 48 / 44; 4096x12288
 # 6-bit 256 rows 73 / 89, 512 rows 149 / 106; 1536x4096 256 rows 20 / 29, 512
-# rows 38 / 35; 8192x8192 256 rows 81 / 116, 384 rows 125 / 110.  From
+# rows 38 / 35; 8192x8192 256 rows 81 / 116, 384 rows 125 / 110.  Wide and
+# expensive matrices leave earlier (gemm_max_rows).  From
 # FUSED_RECONSTRUCT_MIN_ROWS rows the rotations are folded into the
 # reconstructed weight (the reference's rule, exl3.py.lna:184).
 AUTO_RECONSTRUCT_THRESHOLD = 32
@@ -84,6 +85,26 @@ class NullConfig:
 
     class infer_params:
         no_reconstruct = False
+
+
+def gemm_max_rows(k: int, n: int, codebook: int) -> int:
+    """Most rows of a [k] -> [n] linear that the decode GEMM serves faster than the reconstruct path.
+
+    Each of its row tiles (up to 80 rows) decodes the matrix again and leaves
+    fp32 partials of every output, so it loses first where the outputs are many
+    for the weights (us, GEMM / reconstruct: 1024x32768 3-bit 160 rows 46 / 49,
+    161 rows 58 / 53, 256 rows 75 / 61; 512x49152 81 rows 1.06x, 112 rows 0.98x)
+    and where a weight's decode costs more (MUL1, 2048x12288 4-bit: 160 rows
+    1.03x, 192 rows 0.88x), but not where the fp16 weight outgrows the 256 MB
+    cache that the library GEMM reads it back from (4096x32768: 1.02-1.45x at
+    161-256 rows)."""
+    if k < 1024 and n > 32768:
+        return min(GEMM_MAX_ROWS, 80)
+    if n > 16384 and k < 4096 and k * n < 1 << 27:
+        return min(GEMM_MAX_ROWS, 160)
+    if codebook == ops.CB_MUL1 and n >= 8192 and k >= 1024:
+        return min(GEMM_MAX_ROWS, 160)
+    return GEMM_MAX_ROWS
 
 
 class LinearEXL3:
@@ -150,7 +171,7 @@ class LinearEXL3:
         assert x.is_contiguous(), f"LinearEXL3 {self.key}: non-contiguous input {tuple(x.shape)}"
         dtype = out_dtype or self.default_out_dtype
         rows = x.numel() // x.shape[-1]
-        if not params.get("reconstruct") and (rows <= GEMM_MAX_ROWS
+        if not params.get("reconstruct") and (rows <= gemm_max_rows(self.in_features, self.out_features, self.codebook)
                                               or self.config.infer_params.no_reconstruct):
             x2 = x.view(rows, self.in_features)
             if x2.dtype != torch.float16:

@@ -40,6 +40,33 @@ def test_library_exports_every_declared_symbol():
     assert header_symbols() <= exported
 
 
+def _linear_route(monkeypatch, k, n, rows, marker="mcg", params=None):
+    """The path a LinearEXL3.forward call of `rows` rows takes: "decode" or "reconstruct"."""
+    taken = []
+    monkeypatch.setattr(ops, "gemm_into", lambda x, t, u, v, y, cb: taken.append("decode"))
+    monkeypatch.setattr(V.LinearEXL3, "reconstruct_hgemm", lambda self, x, d: taken.append("reconstruct"))
+    lin = V.LinearEXL3(None, k, n, suh=torch.ones(k, dtype=torch.half), svh=torch.ones(n, dtype=torch.half),
+                       trellis=torch.zeros((k // 16, n // 16, 16), dtype=torch.int16),
+                       **({marker: torch.zeros(1, dtype=torch.int32)} if marker else {}))
+    lin.forward(torch.zeros((rows, k), dtype=torch.half), params or {})
+    assert len(taken) == 1
+    return taken[0]
+
+
+@pytest.mark.parametrize("k,n,marker,last", [
+    (256, 1024, "mcg", 256), (1024, 16384, None, 256), (4096, 32768, "mcg", 256), (2048, 65536, "mcg", 256),
+    (1024, 16512, "mcg", 160), (3072, 24576, None, 160), (896, 32768, "mcg", 160),
+    (896, 32896, "mcg", 80), (896, 32896, "mul1", 80),
+    (1024, 8192, "mul1", 160), (896, 8192, "mul1", 256), (4096, 8064, "mul1", 256),
+])
+def test_linear_leaves_the_decode_gemm_by_shape(monkeypatch, k, n, marker, last):
+    """Rows from which a linear takes the reconstruct path, at the edges of the rule."""
+    for rows in (1, 32, 33, last):
+        assert _linear_route(monkeypatch, k, n, rows, marker) == "decode", rows
+    assert _linear_route(monkeypatch, k, n, last + 1, marker) == "reconstruct"
+    assert _linear_route(monkeypatch, k, n, 1, marker, {"reconstruct": True}) == "reconstruct"
+
+
 def test_library_targets_gfx950_only():
     # the code object bundle names its targets; there is exactly one
     blob = open(_lib.LIB_PATH, "rb").read()
