@@ -774,28 +774,36 @@ struct GemmPlan {
 inline GemmPlan gemm_plan(int64_t R, int64_t k, int64_t n, int cus) {
     GemmPlan p;
     p.n_hb = std::max((int)(n / GEMV_COLS), 1);
-    p.n_rt = (int)((R + 16 * GEMM_MAX_RB - 1) / (16 * GEMM_MAX_RB));
-    const int rows = (int)((R + p.n_rt - 1) / p.n_rt);
-    p.rb = (rows + 15) / 16;
-    if (p.rb < 2) p.rb = 2;
     const int S = std::max((int)(k / STEP_K), 1);
-    // k-chunks: whole rounds of one workgroup per CU, each a start (us) and a
-    // step's decode and MFMAs per step of a wave (two waves a SIMD), plus the
-    // partials' way to memory and back.  On 4096x4096, 4096x12288, 1536x4096,
-    // 8192x8192 and 2048x512 at 33-512 rows the count this picks is within 3%
-    // of the best of 1, 2, 3, 4, 6 and 8.
-    const double ts = 0.75 + 0.13 * p.rb;
+    const int rt0 = (int)((R + 16 * GEMM_MAX_RB - 1) / (16 * GEMM_MAX_RB));
+    // Row tiles and k-chunks: whole rounds of one workgroup per CU, each a start
+    // (us) and a step's decode and MFMAs per step of a wave (two waves a SIMD),
+    // plus the partials' way to memory and back.  On 4096x4096, 4096x12288,
+    // 1536x4096, 8192x8192 and 2048x512 at 33-512 rows the k-chunks this picks are
+    // within 3% of the best of 1, 2, 3, 4, 6 and 8.  One row tile more than the
+    // rows need pays where it fills a round that the fewer, taller ones leave
+    // part empty (us, without / with it: 2048x9216 5-bit 81 rows 27.5 / 22.6;
+    // 4096x12288 5-bit 208 rows 82 / 75, where the reconstruct path takes 78); a
+    // gain of less than 5% by this model measured between 0.95x and 1.06x, so it is
+    // not taken.
     double best = 1e30;
-    for (int kc = 1; kc <= 32 && kc <= S; ++kc) {
-        const int ns = (S + kc - 1) / kc, n_kc = (S + ns - 1) / ns;
-        if (n_kc != kc) continue;
-        const int64_t wgs = (int64_t)p.n_hb * GEMV_NCG * p.n_rt * n_kc;
-        const double rounds = (double)((wgs + cus - 1) / cus);
-        const double t = rounds * (1.5 + ts * ((ns + GEMM_NKG - 1) / GEMM_NKG)) + 2e-6 * n_kc * (double)R * (double)n;
-        if (t < best) {
-            best = t;
-            p.nsteps = ns;
-            p.n_kc = n_kc;
+    for (int n_rt = rt0; n_rt <= rt0 + 1; ++n_rt) {
+        const int rows = (int)((R + n_rt - 1) / n_rt), rb = std::max((rows + 15) / 16, 2);
+        const double ts = 0.75 + 0.13 * rb;
+        for (int kc = 1; kc <= 32 && kc <= S; ++kc) {
+            const int ns = (S + kc - 1) / kc, n_kc = (S + ns - 1) / ns;
+            if (n_kc != kc) continue;
+            const int64_t wgs = (int64_t)p.n_hb * GEMV_NCG * n_rt * n_kc;
+            const double rounds = (double)((wgs + cus - 1) / cus);
+            double t = rounds * (1.5 + ts * ((ns + GEMM_NKG - 1) / GEMM_NKG)) + 2e-6 * n_kc * (double)R * (double)n;
+            if (n_rt > rt0) t /= 0.95;
+            if (t < best) {
+                best = t;
+                p.n_rt = n_rt;
+                p.rb = rb;
+                p.nsteps = ns;
+                p.n_kc = n_kc;
+            }
         }
     }
     const int64_t Rp = (int64_t)p.n_rt * 16 * p.rb;

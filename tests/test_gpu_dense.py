@@ -341,6 +341,26 @@ def test_gemm_tile_edges(ops, dev, k, n, bits, rows):
 
 
 @pytest.mark.parametrize("k,n,bits,rows", [
+    (512, 256, 2, 49),        # two row tiles of 2 row blocks where one of 4 would do
+    (1024, 9216, 3, 96),      # three row tiles where two would do, more workgroups than CUs
+    (512, 4096, 3, 144),      # three row tiles of 3 row blocks where two of 5 would do
+    (128, 16384, 4, 80),      # one row tile of 5 row blocks
+])
+def test_gemm_row_tiles(ops, dev, k, n, bits, rows):
+    """The many-row kernel with one row tile more than the rows need, and
+    without, against the oracle on the weights it uses (bound as in
+    test_gemm_tile_edges)."""
+    import torch
+
+    got, _ = _gemm_case(ops, dev, k, n, bits, rows, torch.float32, seed=800 + rows)
+    L = synth.dense(k, n, bits, seed=800 + rows + bits)
+    x = synth.activations(rows, k, seed=800 + 2 * rows)
+    exact = O.linear(x, L["trellis"], L["suh"], L["svh"], bits, O.CB_MCG,
+                     w=O.reconstruct_exact(L["trellis"], bits, O.CB_MCG))
+    assert_close(got, exact, max_abs=2e-5, rel=2e-6, what=f"{k}x{n} K{bits} rows={rows}")
+
+
+@pytest.mark.parametrize("k,n,bits,rows", [
     (512, 33024, 2, 1),       # whole K on four k-groups, two workgroups of some CUs
     (512, 33024, 6, 16),      # the same with a full row block
     (640, 33152, 3, 5),       # 10 steps on four k-groups
