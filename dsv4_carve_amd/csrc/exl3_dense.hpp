@@ -754,13 +754,20 @@ constexpr int GEMM_MAX_RB = 5;      // LDS of the k-groups' exchange: 28 KB per 
 // Rows of one GEMM launch (exl3_gemm runs more rows in slabs of this many).
 constexpr int GEMM_MAX_ROWS = 256;
 
-// Rows that take this path: above 32 all, 17-32 where the columns are many
-// enough that rotating the rows in every column block's workgroups costs more
-// than a launch (32 rows, GEMV / GEMM us: 4096x12288 35 / 26, 8192x8192 35 /
-// 27, but 4096x4096 14.5 / 17).
+// Rows that take this path: above 32 all, 17-32 where a column block's own
+// rotation of the rows, repeated by every one of them, costs more than two more
+// launches.  That work goes with the rows and the weights, and a short K or few
+// columns leave the GEMM's launches idle.  The bound's worst choices over 116
+// matrices of 128-16384 x 1024-65536 at 17-32 rows are within 14% of the better
+// kernel, the mean within 0.2%.  Us, GEMV / GEMM: 4096x4096 6-bit 24 rows 13.3 /
+// 14.0, 32 rows 14.4 / 14.2; 4096x12288 3-bit 17 rows 20.9 / 19.9, 32 rows 26.8 /
+// 19.7; 16384x6144 6-bit 32 rows 52.0 / 32.0; but 256x8192 6-bit 24 rows 7.6 / 9.8
+// and 1024x32768 6-bit 20 rows 14.3 / 17.5.
 // The rotated input's byte offsets are 32-bit.
 inline bool gemm_takes(int64_t m, int64_t k, int64_t n) {
-    return k <= (1 << 20) && (m > GEMV_MAX_ROWS || (m > MAX_ROWS && n >= 8192));
+    if (k > (1 << 20) || m <= MAX_ROWS) return false;
+    if (m > GEMV_MAX_ROWS) return true;
+    return k >= 768 && n > 2048 && (m - 10) * k * n >= (k > 1024 || n <= 16384 ? 250000000 : 900000000);
 }
 
 struct GemmPlan {

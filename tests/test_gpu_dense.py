@@ -316,7 +316,7 @@ def test_xcd_keyed_order_is_bitwise_the_plain_order(ops, dev, monkeypatch, rows)
     (2176, 256, 2, 5),        # 34 steps: a last chunk of 2 steps for 4 k-groups
     (640, 384, 5, 17),        # two row blocks, an odd column-block count
     (4096, 128, 1, 32),       # one column block, every k-chunk on it
-    (256, 8192, 3, 20),       # 17-32 rows on many columns: the many-row kernels
+    (256, 8192, 3, 20),       # 17-32 rows on many columns, a short K
     (128, 128, 4, 33),        # fewer steps than k-groups
     (896, 256, 8, 80),        # a whole row tile of 5 row blocks, 14 steps
     (1152, 384, 7, 81),       # one row more: two row tiles of 3 row blocks
@@ -345,6 +345,9 @@ def test_gemm_tile_edges(ops, dev, k, n, bits, rows):
     (1024, 9216, 3, 96),      # three row tiles where two would do, more workgroups than CUs
     (512, 4096, 3, 144),      # three row tiles of 3 row blocks where two of 5 would do
     (128, 16384, 4, 80),      # one row tile of 5 row blocks
+    (1024, 11008, 3, 32),     # 32 rows just below the many-row kernels' share of the work
+    (1024, 11136, 3, 32),     # and just above
+    (4096, 8832, 2, 17),      # the same at 17 rows
 ])
 def test_gemm_row_tiles(ops, dev, k, n, bits, rows):
     """The many-row kernel with one row tile more than the rows need, and
