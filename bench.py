@@ -378,7 +378,7 @@ LINEAR_ROWS = (32, 64, 144, 512, 2048)
 
 def time_linear(dev, k, n, bits, rows_list, steps=20):
     """us per LinearEXL3.forward call (the plugin's dense entry: the decode
-    GEMV up to its row threshold, the reconstruct path beyond), cold over
+    kernels up to decode_max_rows, the reconstruct path beyond), cold over
     > 512 MB of distinct weight copies, fp16 output."""
     import torch
     from dsv4_carve_amd import ops
@@ -408,7 +408,7 @@ def time_linear(dev, k, n, bits, rows_list, steps=20):
             for i in order:
                 mods[i].forward(x, {}, out_dtype=torch.float16)
         us = replay_median(graph, steps)[0]
-        path = ("gemv" if rows <= V.AUTO_RECONSTRUCT_THRESHOLD else "gemm" if rows <= V.GEMM_MAX_ROWS else
+        path = ("decode" if rows <= V.decode_max_rows(k, n, ops.CB_MCG) else
                 "reconstruct_folded" if rows >= V.FUSED_RECONSTRUCT_MIN_ROWS else "reconstruct")
         res[str(rows)] = {"us": round(us, 2), "path": path,
                           "tflops": round(2.0 * rows * k * n / (us * 1e-6) / 1e12, 1)}

@@ -5,11 +5,11 @@ error behaviour, so the plugin's dispatch code can switch to this package:
 
   * ``LinearEXL3`` / ``make_linear_exl3`` / ``execute_exl3_linear`` -- the
     exllamav3 linear (recipe-lna/exllamav3/exl3.py.lna:16-218,
-    recipe-lna/vllm_exl3_exl3.py.lna:889-926).  Up to AUTO_RECONSTRUCT_THRESHOLD
-    rows run the trellis-decode GEMV kernel, up to GEMM_MAX_ROWS its many-row
-    form; more rows reconstruct the fp16 weight on the GPU and run one hgemm,
-    between row-Hadamard launches below FUSED_RECONSTRUCT_MIN_ROWS rows and on
-    the Hadamard-folded weight from there on.
+    recipe-lna/vllm_exl3_exl3.py.lna:889-926).  Up to decode_max_rows rows (256
+    for most matrices) run the trellis-decode kernels; more rows reconstruct
+    the fp16 weight on the GPU and run one hgemm, between row-Hadamard launches
+    below FUSED_RECONSTRUCT_MIN_ROWS rows and on the Hadamard-folded weight
+    from there on.
   * ``apply_exl3_experts`` and its helpers -- routed experts
     (recipe-lna/vllm_exl3_exl3.py.lna:951-1296, 1543-1569, 1707-1779): backend
     selection by VLLM_EXL3_MOE_KERNEL, strict levels by VLLM_EXL3_MOE_STRICT,
@@ -58,17 +58,18 @@ MUL1_MULTIPLIER = 0x83DCD12D
 MUL1_MARKER_SIGNED_INT32 = -2082680531
 EXL3_SUFFIXES = ("trellis", "suh", "svh", "mcg", "mul1")
 SWIGLU_LIMIT_DEFAULT = 10.0
-# Rows up to AUTO_RECONSTRUCT_THRESHOLD take the decode GEMV (shared scratch,
-# reserved before capture), more the decode GEMM up to GEMM_MAX_ROWS, and the
-# reconstruct path above.  The reference switches at 144 rows
-# (recipe-lna/exllamav3/exl3.py.lna:10).  On MI355X, us per call, GEMM /
+# Where a linear leaves the decode kernels for the reconstruct path
+# (decode_max_rows).  The reference switches at its AUTO_RECONSTRUCT_THRESHOLD
+# of 144 rows (recipe-lna/exllamav3/exl3.py.lna:10); a program that sets the
+# constant of that name to another value than this module's gets that hand-over
+# for every matrix.  At this module's value it is GEMM_MAX_ROWS, or earlier for
+# wide and expensive matrices.  On MI355X, us per call, decode GEMM /
 # reconstruct: 4096x4096 4-bit 256 rows 34 / 40, 384 rows 48 / 44; 4096x12288
 # 6-bit 256 rows 73 / 89, 512 rows 149 / 106; 1536x4096 256 rows 20 / 29, 512
-# rows 38 / 35; 8192x8192 256 rows 81 / 116, 384 rows 125 / 110.  Wide and
-# expensive matrices leave earlier (gemm_max_rows).  From
+# rows 38 / 35; 8192x8192 256 rows 81 / 116, 384 rows 125 / 110.  From
 # FUSED_RECONSTRUCT_MIN_ROWS rows the rotations are folded into the
 # reconstructed weight (the reference's rule, exl3.py.lna:184).
-AUTO_RECONSTRUCT_THRESHOLD = 32
+AUTO_RECONSTRUCT_THRESHOLD = ops.GEMV_MAX_ROWS
 GEMM_MAX_ROWS = 256
 FUSED_RECONSTRUCT_MIN_ROWS = 1024
 MAX_RECONSTRUCT_SLICE_N = 32768
@@ -105,6 +106,13 @@ def gemm_max_rows(k: int, n: int, codebook: int) -> int:
     if codebook == ops.CB_MUL1 and n >= 8192 and k >= 1024:
         return min(GEMM_MAX_ROWS, 160)
     return GEMM_MAX_ROWS
+
+
+def decode_max_rows(k: int, n: int, codebook: int) -> int:
+    """Most rows of a [k] -> [n] linear that the decode kernels serve."""
+    if AUTO_RECONSTRUCT_THRESHOLD != ops.GEMV_MAX_ROWS:
+        return AUTO_RECONSTRUCT_THRESHOLD
+    return gemm_max_rows(k, n, codebook)
 
 
 class LinearEXL3:
@@ -171,8 +179,8 @@ class LinearEXL3:
         assert x.is_contiguous(), f"LinearEXL3 {self.key}: non-contiguous input {tuple(x.shape)}"
         dtype = out_dtype or self.default_out_dtype
         rows = x.numel() // x.shape[-1]
-        if not params.get("reconstruct") and (rows <= gemm_max_rows(self.in_features, self.out_features, self.codebook)
-                                              or self.config.infer_params.no_reconstruct):
+        if not params.get("reconstruct") and (self.config.infer_params.no_reconstruct or rows <= decode_max_rows(
+                self.in_features, self.out_features, self.codebook)):
             x2 = x.view(rows, self.in_features)
             if x2.dtype != torch.float16:
                 x2 = x2.to(torch.float16)
@@ -1533,11 +1541,11 @@ class Exl3LinearMethod:
     @staticmethod
     def _prewarm(layer) -> None:
         """Reserve the shared scratch of every call this module can make before
-        any graph capture: each shard's GEMV for every row count it takes (up
-        to AUTO_RECONSTRUCT_THRESHOLD rows, whatever LNA_EXL3_PREWARM_ROWS
+        any graph capture: each shard's decode kernels for every row count that
+        uses it (up to ops.GEMV_MAX_ROWS rows, whatever LNA_EXL3_PREWARM_ROWS
         says: a capture at a row count without an earlier eager call would
-        otherwise need a larger buffer), and the fused group at its row counts
-        (up to DENSE_GROUP_MAX_ROWS)."""
+        otherwise need a larger buffer; more rows bring their own), and the
+        fused group at its row counts (up to DENSE_GROUP_MAX_ROWS)."""
         lins = [lin for lin in layer._exl3_linears if lin is not None]
         if not lins or lins[0].trellis.device.type != "cuda":
             return
@@ -1545,7 +1553,7 @@ class Exl3LinearMethod:
         try:
             before = _vram_mark(dev)
             for lin in lins:
-                ops.prepare_gemm(dev, AUTO_RECONSTRUCT_THRESHOLD, int(lin.in_features), int(lin.out_features))
+                ops.prepare_gemm(dev, ops.GEMV_MAX_ROWS, int(lin.in_features), int(lin.out_features))
             _vram_report("registration.gemv_scratch", getattr(layer, "prefix", "?"), before, _vram_mark(dev))
             prewarm_exl3_dense_group(layer)
         except Exception as exc:

@@ -8,6 +8,7 @@ import ctypes
 import os
 import re
 import subprocess
+import types
 
 import numpy as np
 import pytest
@@ -65,6 +66,23 @@ def test_linear_leaves_the_decode_gemm_by_shape(monkeypatch, k, n, marker, last)
         assert _linear_route(monkeypatch, k, n, rows, marker) == "decode", rows
     assert _linear_route(monkeypatch, k, n, last + 1, marker) == "reconstruct"
     assert _linear_route(monkeypatch, k, n, 1, marker, {"reconstruct": True}) == "reconstruct"
+
+
+@pytest.mark.parametrize("threshold", [8, 144, 400])
+def test_reconstruct_threshold_set_by_a_program(monkeypatch, threshold):
+    """AUTO_RECONSTRUCT_THRESHOLD at another value than the module's is the last
+    row count of the decode kernels, below and above the module's own limits,
+    and the prewarm still reserves what every decode call of 1-32 rows uses."""
+    monkeypatch.setattr(V, "AUTO_RECONSTRUCT_THRESHOLD", threshold)
+    for k, n in ((256, 1024), (1024, 16512)):
+        assert _linear_route(monkeypatch, k, n, threshold) == "decode"
+        assert _linear_route(monkeypatch, k, n, threshold + 1) == "reconstruct"
+    reserved = []
+    monkeypatch.setattr(ops, "prepare_gemm", lambda dev, rows, k, n: reserved.append((rows, k, n)))
+    lin = types.SimpleNamespace(trellis=types.SimpleNamespace(device=torch.device("cuda", 0)), in_features=512,
+                                out_features=256)
+    V.Exl3LinearMethod._prewarm(types.SimpleNamespace(_exl3_linears=[lin], _exl3_dense_group=None))
+    assert reserved == [(ops.GEMV_MAX_ROWS, 512, 256)]
 
 
 def test_library_targets_gfx950_only():
