@@ -52,6 +52,19 @@ def _check(cond: bool, msg: str) -> None:
 
 # ------------------------------------------------------------------ shared scratch
 
+def _block_bytes(buf: torch.Tensor) -> int:
+    """Size of the allocator's block that starts at `buf` (its own size if the allocator lists none)."""
+    ptr = buf.data_ptr()
+    for segment in torch.cuda.memory_snapshot():
+        address = segment["address"]
+        if segment["device"] == buf.device.index and address <= ptr < address + segment["total_size"]:
+            for block in segment["blocks"]:
+                if address == ptr:
+                    return int(block["size"])
+                address += block["size"]
+    return buf.numel()
+
+
 class _ScratchPool:
     """One zeroed scratch buffer per (device, purpose), grown outside capture.
 
@@ -96,21 +109,29 @@ class _ScratchPool:
 
     @staticmethod
     def _allocate(nbytes: int, device: torch.device) -> torch.Tensor:
-        """A zeroed buffer in a block of its own size.
+        """A zeroed buffer, in a block of its own size where the allocator has one.
 
-        The allocator hands out a cached block whole where less than 1 MiB of
-        it would be left over, and a buffer of this pool would keep that excess
-        for the process's life.  Such a block is set aside while another is
-        asked for (a few times at most; a buffer of more than 32 MiB takes what
-        it gets)."""
-        aside = []
-        while device.type == "cuda" and nbytes <= 32 << 20 and len(aside) < 8:
-            before = torch.cuda.memory_allocated(device)
-            buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            if torch.cuda.memory_allocated(device) - before < nbytes + 512:
-                return buf.zero_()
+        Of 1 to 10 MiB the allocator hands out a cached block whole where less
+        than 1 MiB of it would be left over, and a buffer of this pool would keep
+        that excess for the process's life.  Such a block is set aside while the
+        next is asked for: each is one the allocator held already (a fresh segment
+        of these sizes always splits), and the first serves if there is no room for
+        another.  Smaller sizes always split, and larger ones get the same excess
+        from a fresh segment."""
+        aside: list[torch.Tensor] = []
+        while True:
+            try:
+                buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:
+                if not aside:
+                    raise
+                buf = aside[0]
+                break
+            if (device.type != "cuda" or not 1 << 20 < nbytes < 10 << 20 or len(aside) == 16
+                    or _block_bytes(buf) < nbytes + 512):
+                break
             aside.append(buf)
-        return torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        return buf.zero_()
 
     def current(self, device: torch.device, purpose: str) -> torch.Tensor | None:
         idx = device.index if device.index is not None else torch.cuda.current_device()

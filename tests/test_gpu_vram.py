@@ -238,3 +238,45 @@ def test_scratch_takes_no_oversized_cached_block(mib):
     buf = ops.SCRATCH._allocate(nbytes, dev)
     grown = torch.cuda.memory_allocated(dev) - before
     assert nbytes <= grown < nbytes + 512 and int(buf.count_nonzero()) == 0
+
+
+def test_scratch_of_a_segment_of_its_own_is_asked_for_once():
+    """11.5 MiB gets a segment of its own, rounded up to 12 MiB and not split:
+    the buffer takes it, and nothing more is reserved."""
+    import torch
+
+    from dsv4_carve_amd import ops
+
+    dev = torch.device("cuda", 0)
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_reserved(dev)
+    buf = ops.SCRATCH._allocate(23 << 19, dev)
+    assert torch.cuda.memory_reserved(dev) - before <= 12 << 20 and int(buf.count_nonzero()) == 0
+
+
+def test_scratch_takes_an_oversized_block_where_nothing_else_fits():
+    """With no memory left to reserve, a block that is a little too large serves."""
+    import torch
+
+    from dsv4_carve_amd import ops
+
+    dev = torch.device("cuda", 0)
+    torch.cuda.empty_cache()
+    nbytes, mib3 = 9 << 18, 3 << 20
+    held = {}
+    total = torch.cuda.get_device_properties(dev).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(dev) + (48 << 20)) / total, dev)
+        for size in (mib3, nbytes):                   # every place that is left, two fresh segments among them
+            with pytest.raises(torch.OutOfMemoryError):
+                while True:
+                    t = torch.empty(size, dtype=torch.uint8, device=dev)
+                    held[t.data_ptr()] = t
+        # one block between two that stay
+        hole = next(p for p, t in held.items() if t.numel() == mib3
+                    and all(q in held and held[q].numel() == mib3 for q in (p - mib3, p + mib3)))
+        del t, held[hole]
+        buf = ops.SCRATCH._allocate(nbytes, dev)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, dev)
+    assert buf.data_ptr() == hole and ops._block_bytes(buf) == mib3 and int(buf.count_nonzero()) == 0
