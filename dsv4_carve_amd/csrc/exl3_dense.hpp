@@ -524,6 +524,24 @@ __device__ __forceinline__ void load_quarter(QuarterTile<BITS>& d, gptr_t<uint32
     load_words_g<BITS + 1>(d.w + 4 * BITS - 1, t + (p + 4) * BITS - 1);
 }
 
+// decode_pair on a quarter tile: every word it can read has been loaded.
+template <int BITS>
+constexpr bool quarter_holds(int w) {
+    return w < BITS || (w >= 4 * BITS - 1 && w < 5 * BITS) || w == 8 * BITS - 1;
+}
+template <int BITS, int T>
+constexpr bool quarter_window() {          // the words of element T's window
+    using S = WinSel<BITS, T>;
+    return quarter_holds<BITS>(S::I1) && (S::O >= 16 || quarter_holds<BITS>((S::I1 + 8 * BITS - 1) % (8 * BITS)));
+}
+template <int BITS, int CB, int T>
+__device__ __forceinline__ uint32_t decode_quarter(const QuarterTile<BITS>& t) {
+    static_assert(quarter_window<BITS, T>() && quarter_window<BITS, WinSel<BITS, T>::SRC_T>() &&
+                      quarter_holds<BITS>(null_word<BITS, T>()),
+                  "a word that load_quarter leaves out");
+    return decode_pair<BITS, CB, T>(t.w);
+}
+
 // The lane's MFMA columns in decode order: columns n and n + 8, whose eight
 // windows at one k-group are consecutive in the stream, back to back.
 __host__ __device__ constexpr int quarter_col(int j) { return 4 * (j >> 1) + 8 * (j & 1); }
@@ -616,10 +634,10 @@ __device__ __forceinline__ void gemv_item(const uint16_t* __restrict__ x, const 
                 constexpr int r = decltype(RI)::value;
                 constexpr int T0 = 32 * (n & 7) + 8 * r + 4 * (n >> 3);
                 u32x4_t b;
-                b[0] = decode_pair<BITS, CB, T0 + 0>(t.w);
-                b[1] = decode_pair<BITS, CB, T0 + 1>(t.w);
-                b[2] = decode_pair<BITS, CB, T0 + 2>(t.w);
-                b[3] = decode_pair<BITS, CB, T0 + 3>(t.w);
+                b[0] = decode_quarter<BITS, CB, T0 + 0>(t);
+                b[1] = decode_quarter<BITS, CB, T0 + 1>(t);
+                b[2] = decode_quarter<BITS, CB, T0 + 2>(t);
+                b[3] = decode_quarter<BITS, CB, T0 + 3>(t);
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
                     acc[rb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[rb][r], __builtin_bit_cast(half8_t, b),
@@ -918,10 +936,10 @@ __global__ __launch_bounds__(WAVE * GEMM_NKG) void gemm_kernel(
                 constexpr int q = decltype(JI)::value, n = quarter_col(q);
                 constexpr int T0 = 32 * (n & 7) + 8 * r + 4 * (n >> 3);
                 u32x4_t b;
-                b[0] = decode_pair<BITS, CB, T0 + 0>(t.w);
-                b[1] = decode_pair<BITS, CB, T0 + 1>(t.w);
-                b[2] = decode_pair<BITS, CB, T0 + 2>(t.w);
-                b[3] = decode_pair<BITS, CB, T0 + 3>(t.w);
+                b[0] = decode_quarter<BITS, CB, T0 + 0>(t);
+                b[1] = decode_quarter<BITS, CB, T0 + 1>(t);
+                b[2] = decode_quarter<BITS, CB, T0 + 2>(t);
+                b[3] = decode_quarter<BITS, CB, T0 + 3>(t);
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
                     acc[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[r][rb], __builtin_bit_cast(half8_t, b),

@@ -94,9 +94,18 @@ __device__ __forceinline__ uint32_t win16(const uint32_t* W) {
 #define EXL3_NULL_DECODE 0
 #endif
 
+// The word that stands for element T: one its window lies in, the earlier where
+// it straddles two, so a kernel that loads only its windows' words (the quarter
+// tiles) has loaded it, and every word loaded is read by some element.
+template <int BITS, int T>
+constexpr int null_word() {
+    using S = WinSel<BITS, T>;
+    return S::O >= 16 ? S::I1 : (S::I1 + 8 * BITS - 1) % (8 * BITS);
+}
+
 template <int BITS, int CB, int T>
 __device__ __forceinline__ uint32_t decode_pair(const uint32_t* W) {
-    if constexpr (EXL3_NULL_DECODE) return W[T % (8 * BITS)];
+    if constexpr (EXL3_NULL_DECODE) return W[null_word<BITS, T>()];
     else if constexpr (CB == CB_MUL1) return codebook_pair<CB, WinSel<BITS, T>::HI>(win_src<BITS, T>(W));
     else return codebook_word<CB>(win16<BITS, T>(W));
 }
