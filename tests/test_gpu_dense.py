@@ -340,6 +340,25 @@ def test_gemm_tile_edges(ops, dev, k, n, bits, rows):
     assert_close(got, exact, max_abs=2e-5, rel=2e-6, what=f"{k}x{n} K{bits} rows={rows} (exact addends)")
 
 
+@pytest.mark.parametrize("cb", [O.CB_3INST, O.CB_MUL1])
+@pytest.mark.parametrize("bits", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("rows", [3, 20, 80, 160])
+def test_dense_kernels_other_codebooks(ops, dev, rows, bits, cb):
+    """Each dense kernel (one and two row blocks of the GEMV, one row tile and
+    several of the many-row kernels) with the 3INST and MUL1 codebooks, at the
+    widths where MUL1's windows share a funnel in pairs and one where they do
+    not, against the oracle on the weights they use (bound as in
+    test_gemm_tile_edges)."""
+    import torch
+
+    k, n = 640, 384
+    got, _ = _gemm_case(ops, dev, k, n, bits, rows, torch.float32, seed=900 + rows, cb=cb)
+    L = synth.dense(k, n, bits, seed=900 + rows + bits)
+    x = synth.activations(rows, k, seed=900 + 2 * rows)
+    exact = O.linear(x, L["trellis"], L["suh"], L["svh"], bits, cb, w=O.reconstruct_exact(L["trellis"], bits, cb))
+    assert_close(got, exact, max_abs=2e-5, rel=2e-6, what=f"{k}x{n} K{bits} rows={rows} cb={cb}")
+
+
 @pytest.mark.parametrize("k,n,bits,rows", [
     (512, 256, 2, 49),        # two row tiles of 2 row blocks where one of 4 would do
     (1024, 9216, 3, 96),      # three row tiles where two would do, more workgroups than CUs
