@@ -20,6 +20,7 @@ EXPORTS = (
     "exl3_had_rows",
     "exl3_gemm_scratch_bytes",
     "exl3_gemm",
+    "exl3_gemm_rows",
     "exl3_gemm_group_scratch_bytes",
     "exl3_gemm_group",
     "exl3_moe_scratch_bytes",
@@ -52,6 +53,7 @@ _SIGS = {
     "exl3_had_rows": ([_P, _I, _P, _I, _L, _L, _P, _P, _F, _P], _I),
     "exl3_gemm_scratch_bytes": ([_L, _L, _L], _L),
     "exl3_gemm": ([_P, _L, _L, _P, _L, _I, _I, _P, _P, _P, _I, _P, _L, _P], _I),
+    "exl3_gemm_rows": ([_P, _I, _L, _L, _P, _L, _I, _I, _P, _P, _P, _I, _P, _L, _P], _I),
     "exl3_gemm_group_scratch_bytes": ([_L, _L, _L, _P], _L),
     "exl3_gemm_group": ([_P, _L, _L, _L, _P, _P, _P, _P, _P, _I, _P, _I, _P, _L, _P], _I),
     "exl3_moe_scratch_bytes": ([_L, _L, _L], _L),

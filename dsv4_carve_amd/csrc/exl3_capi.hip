@@ -49,8 +49,8 @@ static int dequant_impl(const int16_t* trellis, int64_t k, int64_t n, int bits, 
     return 0;
 }
 
-// Rows [0, R), R <= GEMM_MAX_ROWS, by the GEMM kernels.
-static int gemm_slab(const uint16_t* a, int R, int64_t k, const int16_t* b, int64_t n, int bits, int codebook,
+// Rows [0, R), R <= GEMM_MAX_ROWS, of a's own type, by the GEMM kernels.
+static int gemm_slab(const void* a, int a_kind, int R, int64_t k, const int16_t* b, int64_t n, int bits, int codebook,
                      const uint16_t* suh, const uint16_t* svh, void* c, int c_kind, void* scratch, int cus,
                      hipStream_t s) {
     const GemmPlan g = gemm_plan(R, k, n, cus);
@@ -58,7 +58,10 @@ static int gemm_slab(const uint16_t* a, int R, int64_t k, const int16_t* b, int6
     float4_t* partials = reinterpret_cast<float4_t*>(reinterpret_cast<char*>(scratch) + align_up(g.xd_bytes, 256));
     const bool xcd = xcd_order_allowed() && g.n_hb % N_XCD == 0;
     const int64_t waves = (int64_t)(R + 3) / 4 * (k / 128);
-    hipLaunchKernelGGL(gemm_rotate_kernel<0>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, a, suh, R, (int)k,
+    const auto rotate = a_kind == OUT_F32    ? gemm_rotate_kernel<OUT_F32>
+                        : a_kind == OUT_BF16 ? gemm_rotate_kernel<OUT_BF16>
+                                             : gemm_rotate_kernel<OUT_F16>;
+    hipLaunchKernelGGL(rotate, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, a, suh, R, (int)k,
                        g.n_rt * 16 * g.rb, xd);
     int rc = check_launch();
     if (rc) return rc;
@@ -132,7 +135,7 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
         void* cr = reinterpret_cast<char*>(c) + (size_t)r0 * n * c_elem;
         int rc = 0;
         if (gemm_takes(R, k, n)) {
-            if ((rc = gemm_slab(ar, R, k, b, n, bits, codebook, suh, svh, cr, c_kind, scratch, cus, s))) return rc;
+            if ((rc = gemm_slab(ar, OUT_F16, R, k, b, n, bits, codebook, suh, svh, cr, c_kind, scratch, cus, s))) return rc;
             continue;
         }
         const GemvPlan p = gemv_plan(R, k, n, cus);
@@ -147,6 +150,24 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
         }
     }
     return 0;
+}
+
+int exl3_gemm_rows(const void* a, int a_kind, int64_t m, int64_t k, const int16_t* b, int64_t n, int bits,
+                   int codebook, const uint16_t* suh, const uint16_t* svh, void* c, int c_kind, void* scratch,
+                   int64_t scratch_bytes, void* stream) {
+    clear_error();
+    if (!a || !b || !c || !suh || !svh || !scratch) return fail("null pointer");
+    if (a_kind < OUT_F16 || a_kind > OUT_F32) return fail("a_kind must be 0 (fp16), 1 (bf16) or 2 (fp32)");
+    if (m <= GEMV_MAX_ROWS || m > GEMM_MAX_ROWS) return fail("m must be in 33..256");
+    if (codebook < CB_3INST || codebook > CB_MUL1) return fail("codebook must be 0 (3inst), 1 (mcg) or 2 (mul1)");
+    if (k <= 0 || k % 128) return fail("k must be a positive multiple of 128");
+    if (n <= 0 || n % 128) return fail("n must be a positive multiple of 128");
+    if (!gemm_takes(m, k, n)) return fail("k must be at most 2^20");
+    if (c_kind < OUT_F16 || c_kind > OUT_F32) return fail("c_kind must be 0 (fp16), 1 (bf16) or 2 (fp32)");
+    const int cus = device_cus();
+    if (scratch_bytes < dense_scratch_bytes(m, k, n, cus)) return fail("scratch too small");
+    return gemm_slab(a, a_kind, (int)m, k, b, n, bits, codebook, suh, svh, c, c_kind, scratch, cus,
+                     reinterpret_cast<hipStream_t>(stream));
 }
 
 // Scratch of exactly this fan call: per member, its split-K partials

@@ -190,8 +190,12 @@ def _gemm_impl(a, b, c, suh, svh, codebook, scratch):
     m, k = a.shape
     n = b.shape[1] * 16
     bits = b.shape[2] // 16
-    _lib.check(L.exl3_gemm(_ptr(a), m, k, _ptr(b), n, bits, int(codebook), _ptr(suh), _ptr(svh),
-                           _ptr(c), OUT_KIND[c.dtype], _ptr(scratch), scratch.numel(), _stream(a.device)))
+    rest = (m, k, _ptr(b), n, bits, int(codebook), _ptr(suh), _ptr(svh), _ptr(c), OUT_KIND[c.dtype], _ptr(scratch),
+            scratch.numel(), _stream(a.device))
+    if a.dtype == torch.float16:
+        _lib.check(L.exl3_gemm(_ptr(a), *rest))
+    else:
+        _lib.check(L.exl3_gemm_rows(_ptr(a), OUT_KIND[a.dtype], *rest))
 
 
 def _route_args(ids, w, emap):
@@ -375,8 +379,25 @@ def prepare_gemm(device: torch.device, max_rows: int, k: int, n: int) -> None:
 def gemm_into(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
               c: torch.Tensor, codebook: int = CB_MCG) -> torch.Tensor:
     """c = had_out(had_in(x*suh) @ Wq) * svh for x fp16 [m, k]; c fp16/bf16/fp32 [m, n]."""
-    bits = _check_trellis(trellis)
+    _check_trellis(trellis)
     _check(x.dim() == 2 and x.dtype == torch.float16 and x.is_contiguous(), "x must be contiguous fp16 [m, k]")
+    return _gemm_call(x, trellis, suh, svh, c, codebook)
+
+
+GEMM_ROWS = range(GEMV_MAX_ROWS + 1, 257)
+
+
+def gemm_rows_into(x: torch.Tensor, trellis: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
+                   c: torch.Tensor, codebook: int = CB_MCG) -> torch.Tensor:
+    """gemm_into on x.half(), for a GEMM_ROWS count of fp16, bf16 or fp32 rows and k <= 2**20, without the cast's
+    launch."""
+    _check_trellis(trellis)
+    _check(x.dim() == 2 and x.dtype in OUT_KIND and x.is_contiguous(), "x must be contiguous fp16, bf16 or fp32 [m, k]")
+    _check(x.shape[0] in GEMM_ROWS, "x must have 33 to 256 rows")
+    return _gemm_call(x, trellis, suh, svh, c, codebook)
+
+
+def _gemm_call(x, trellis, suh, svh, c, codebook):
     m, k = x.shape
     n = trellis.shape[1] * 16
     _check(k == trellis.shape[0] * 16, "x feature dimension does not match trellis")

@@ -182,11 +182,15 @@ class LinearEXL3:
         if not params.get("reconstruct") and (self.config.infer_params.no_reconstruct or rows <= decode_max_rows(
                 self.in_features, self.out_features, self.codebook)):
             x2 = x.view(rows, self.in_features)
+            gemm = ops.gemm_into
             if x2.dtype != torch.float16:
-                x2 = x2.to(torch.float16)
+                if x2.dtype in ops.OUT_KIND and rows in ops.GEMM_ROWS and self.in_features <= 1 << 20:
+                    gemm = ops.gemm_rows_into
+                else:
+                    x2 = x2.to(torch.float16)
             y = torch.empty((rows, self.out_features), dtype=dtype if dtype in ops.OUT_KIND else torch.float32,
                             device=x.device)
-            ops.gemm_into(x2, self.trellis, self.suh, self.svh, y, self.codebook)
+            gemm(x2, self.trellis, self.suh, self.svh, y, self.codebook)
             if y.dtype != dtype:
                 y = y.to(dtype)
             if self.bias is not None:

@@ -79,6 +79,15 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
               void* scratch, int64_t scratch_bytes, void* stream);
 
 /*
+ * exl3_gemm of 33..256 rows with a of its own type (a_kind 0 = fp16, 1 = bf16,
+ * 2 = fp32; k <= 2^20): a is read as its values rounded to fp16, so the result is
+ * bitwise exl3_gemm's on that cast.  Same scratch.
+ */
+int exl3_gemm_rows(const void* a, int a_kind, int64_t m, int64_t k, const int16_t* b, int64_t n, int bits,
+                   int codebook, const uint16_t* suh, const uint16_t* svh, void* c, int c_kind,
+                   void* scratch, int64_t scratch_bytes, void* stream);
+
+/*
  * Same-input fan: c_j[m][n_j] = had_out(had_in(a . suh_j) . Wq_j) . svh_j for
  * count (1..8) matrices that read one input a (fp16 [m][k], k % 128 == 0): one
  * launch of split-K partial sums over every member per bit width present, one

@@ -423,6 +423,56 @@ def test_gemm_unaligned_operands(ops, dev, rows):
         assert torch.equal(got, want), dt
 
 
+@pytest.mark.parametrize("k,n,rows", [(512, 256, 33), (896, 384, 161), (128, 128, 256)])
+def test_many_rows_of_other_types_are_the_cast_ones(ops, dev, k, n, rows):
+    """bf16 and fp32 rows on the many-row kernels give bitwise what their fp16
+    cast gives: normal, subnormal and overflowing values, infinities and NaN
+    among them, at odd addresses of their type too; other row counts are
+    refused."""
+    import torch
+
+    L = synth.dense(k, n, 3, seed=61)
+    t, u, v = (to_dev(L[key], dev) for key in ("trellis", "suh", "svh"))
+    x = torch.randn((rows, k), generator=torch.Generator().manual_seed(62)).to(dev)
+    x[1] *= 1e-6                                       # subnormal in fp16
+    x[2] += 65519.0                                    # at fp16's largest value, some above
+    x[3, 5], x[4, 7], x[5, 9] = float("inf"), float("-inf"), float("nan")
+    for dt in (torch.bfloat16, torch.float32):
+        xd = x.to(dt)
+        want = ops.gemm(xd.half(), t, u, v, ops.CB_MCG, torch.float32)
+        buf = torch.empty(rows * k + 1, dtype=dt, device=dev)
+        buf[1:] = xd.reshape(-1)
+        for a in (xd, buf[1:].view(rows, k)):
+            got = ops.gemm_rows_into(a, t, u, v, torch.empty_like(want))
+            assert torch.equal(got.isnan(), want.isnan())
+            assert torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0)), dt
+        assert torch.isfinite(want[6:]).all() and not torch.isfinite(want[3:6]).all()
+        for bad in (xd[:32], torch.cat([xd] * 9)[:257]):
+            with pytest.raises(RuntimeError, match="33 to 256 rows"):
+                ops.gemm_rows_into(bad, t, u, v, torch.empty((bad.shape[0], n), device=dev))
+
+
+def test_many_row_linear_reads_its_input_type(dev):
+    """A linear of 33-256 bf16 or fp32 rows launches no cast, and gives the
+    bits of the cast input's call."""
+    import torch
+
+    from dsv4_carve_amd import vllm_exl3 as V
+
+    L = synth.dense(512, 384, 4, seed=63)
+    mcg = torch.tensor([V.MCG_MARKER_SIGNED_INT32], dtype=torch.int32, device=dev)
+    lin = V.make_linear_exl3(*(to_dev(L[key], dev) for key in ("trellis", "suh", "svh")), mcg)
+    for rows in (32, 33, 256):
+        for dt in (torch.bfloat16, torch.float32):
+            x = to_dev(synth.activations(rows, 512, seed=64), dev).to(dt)
+            want = lin.forward(x.half(), {}, out_dtype=torch.float32)
+            held = torch.cuda.memory_stats(dev)["allocation.all.allocated"]
+            got = lin.forward(x, {}, out_dtype=torch.float32)
+            allocated = torch.cuda.memory_stats(dev)["allocation.all.allocated"] - held
+            assert torch.equal(got, want)
+            assert allocated == 2, "the output and, up to 32 rows, the cast, above, the call's scratch"
+
+
 def test_many_row_linear_captures_without_prewarm(dev):
     """A linear of more than 32 rows captured with no earlier call (its scratch
     is the call's own) replays bitwise what the eager call gives, with other

@@ -270,6 +270,19 @@ def test_gemm_group_argument_errors_without_device(m, k, ns, msg):
     assert msg in _err()
 
 
+@pytest.mark.parametrize("change,msg", [
+    ({"m": 32}, "33..256"), ({"m": 257}, "33..256"), ({"a_kind": 3}, "a_kind"), ({"k": 192}, "k must"),
+    ({"k": (1 << 20) + 128}, "2^20"), ({"n": 0}, "n must"), ({"cb": 3}, "codebook"), ({"c_kind": 3}, "c_kind"),
+    ({"scratch_bytes": 1024}, "scratch too small"), ({"scratch": None}, "null"),
+])
+def test_gemm_rows_argument_errors_without_device(change, msg):
+    p = ctypes.c_void_p(16)
+    v = dict(a_kind=1, m=33, k=256, n=128, bits=3, cb=1, c_kind=2, scratch=p, scratch_bytes=1 << 40) | change
+    assert _lib.load().exl3_gemm_rows(p, v["a_kind"], v["m"], v["k"], p, v["n"], v["bits"], v["cb"], p, p, p,
+                                      v["c_kind"], v["scratch"], v["scratch_bytes"], None) == -1
+    assert msg in _err()
+
+
 def test_gemm_group_width_and_kind_errors_without_device():
     lib = _lib.load()
     arr = (ctypes.c_int64 * 2)(256, 512)
