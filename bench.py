@@ -991,6 +991,27 @@ def cpu_baseline(rows: int, bits: list[int], seed: int, us_ids: np.ndarray) -> d
 EXTRA_LEGS = ("ceiling", "null", "sweep", "rows17", "tp8", "prefill", "stack", "dense", "fan", "glue")
 
 
+MAX_LINE = 12000        # bytes of the JSON line; a reader that keeps the last 16 KB of stdout has it whole
+
+
+def json_line(line: dict, extra: dict) -> str:
+    """The result line: `line`, then the extra legs' fields that fit in MAX_LINE bytes, smallest first; the others go
+    to stderr, one JSON object each, and are named in `on_stderr`."""
+    pack = lambda d: json.dumps(d, separators=(",", ":"))
+    out, left = dict(line), []
+    room = MAX_LINE - len(pack(line)) - len(pack({"on_stderr": list(extra)}))
+    for size, key in sorted((len(pack({k: v})), k) for k, v in extra.items()):
+        if size <= room:
+            room -= size
+            out[key] = extra[key]
+        else:
+            left.append(key)
+            print(pack({key: extra[key]}), file=sys.stderr, flush=True)
+    if left:
+        out["on_stderr"] = left
+    return pack(out)
+
+
 def main() -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1251,8 +1272,7 @@ def main() -> int:
         "latency_per_call": latency,
         "cpu_baseline": cpu,
     }
-    line.update(extra)
-    print(json.dumps(line))
+    print(json_line(line, extra))
     return 0
 
 

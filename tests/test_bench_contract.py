@@ -4,6 +4,7 @@ the actual synthetic tensors, not against the formula)."""
 
 from __future__ import annotations
 
+import json
 import os
 import subprocess
 import sys
@@ -47,3 +48,17 @@ def test_step_bytes_count_each_distinct_valid_expert_once():
     ids = np.array([[0, 1, 1], [1, 3, -1], [7, 0, 3]])          # 0, 1, 3 valid; -1 and 7 are not
     want = sum(bench.expert_bytes(h, i, bits[e]) for e in (0, 1, 3)) + 3 * h * (2 + 4)
     assert bench.step_bytes(ids, bits, h, i) == want
+
+
+def test_result_line_fits_and_names_what_it_leaves_out(capsys):
+    line = {"metric": "m", "value": 1.5, "config": {"rows": 16}}
+    extra = {"a": {"us": 1.0}, "sweep": {str(i): {"us": 10.25, "GBps": 301.5} for i in range(400)},
+             "dense": {str(i): {"us": 10.25} for i in range(600)}, "b": [1, 2]}
+    text = bench.json_line(line, extra)
+    assert len(text) <= bench.MAX_LINE and "\n" not in text
+    got = json.loads(text)
+    assert {k: got[k] for k in line} == line and got["a"] == extra["a"] and got["b"] == extra["b"]
+    err = [json.loads(l) for l in capsys.readouterr().err.splitlines()]
+    assert [list(d)[0] for d in err] == got["on_stderr"]
+    assert {k: v for d in err for k, v in d.items()} | {k: got[k] for k in extra if k in got} == extra
+    assert json.loads(bench.json_line(line, {"a": 1})) == line | {"a": 1}
