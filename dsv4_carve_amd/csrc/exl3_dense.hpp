@@ -345,9 +345,9 @@ __global__ __launch_bounds__(64) void had_rows_kernel(const void* x, int x_kind,
 // rotated 1.9, weights 2.45 (at memory rate), decoded and multiplied 4.7, sums
 // stored 5.5, plus two launches.  Against 256-column items of 128 k-rows on four
 // waves that each decode a quarter of every whole tile (us per call in a graph,
-// before / now): 4096x4096 6-bit 1 row 10.3 / 9.6, 16 rows 13.5 / 11.2, 32 rows
-// 18.2 / 14.5; 4096x1536 3-bit 16 rows 11.1 / 8.8; 4096x12288 4-bit 1 row 17.4 /
-// 15.2; 8192x8192 3-bit 16 rows 26.2 / 21.5; 2048x2048 2-bit 1 row 7.6 / 6.2.
+// before / now): 4096x4096 6-bit 1 row 10.4 / 9.5, 16 rows 13.3 / 11.0;
+// 4096x1536 3-bit 16 rows 11.2 / 8.7; 4096x12288 4-bit 1 row 17.6 / 13.8;
+// 8192x8192 3-bit 16 rows 25.7 / 20.6; 2048x2048 2-bit 1 row 7.6 / 5.9.
 //
 // The rotated input is kept in LDS with every half doubled, so an MFMA's A
 // operand is one 16-byte read.
@@ -760,11 +760,11 @@ __global__ __launch_bounds__(64) void gemv_reduce_kernel(const float* __restrict
 //
 // What it replaces above 32 rows is the reconstructed weight in memory and a
 // library GEMM between two row-Hadamard launches.  Us per call, before / with
-// this kernel (bf16 out): 4096x4096 at 4 bits, 33 rows 31.7 / 16.9, 72 rows
-// 34.9 / 20.1, 128 rows 40.4 / 23.3, 256 rows 40.3 / 34.0; 4096x12288 at 6
-// bits, 72 rows 65.8 / 32.2, 256 rows 89.4 / 73.2; 1536x4096 at 3 bits, 256
-// rows 28.9 / 19.8.  From 384 rows the reconstructed weight is read often
-// enough to win (4096x4096 44.1 / 48, 512 rows 49.4 / 64.5).
+// this kernel (fp16 in, bf16 out): 4096x4096 at 4 bits, 33 rows 29.7 / 15.4, 72
+// rows 32.8 / 18.2, 128 rows 38.1 / 21.2, 256 rows 37.6 / 31.2; 4096x12288 at 6
+// bits, 72 rows 65.3 / 33, 256 rows 87 / 76; 1536x4096 at 3 bits, 256 rows 28.1 /
+// 19.1.  From 384 rows the reconstructed weight is read often enough to win
+// (4096x4096 at 6 bits 42 / 49).
 
 constexpr int GEMM_NKG = 8;
 constexpr int GEMM_MAX_RB = 5;      // LDS of the k-groups' exchange: 28 KB per row block

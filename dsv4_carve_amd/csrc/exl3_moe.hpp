@@ -845,8 +845,8 @@ __device__ __forceinline__ bool slot_group(const Params& P, int o, SlotGroup& g,
 // rotates the gate column block, the upper the up one, each with all its chunk
 // loads in flight (up to 32), then a row swap gives both halves both values.
 // For calls of one row with chunks of one block, where down_input_chunk would
-// leave a half-wave idle and double the chain (256-expert layer 45.3 -> 44.6 us,
-// TP slice 23.3 -> 22.2).  With more units both half-waves have one of their own
+// leave a half-wave idle and double the chain (256-expert layer 45.3 -> 44.1 us,
+// TP slice 23.6 -> 21.8).  With more units both half-waves have one of their own
 // and splitting each loses (16 rows on hot experts of 32: 44 -> 59 us), and both
 // forms in one kernel cost its other items 1-2%, so it is an instance of its own.
 __device__ __forceinline__ void down_input_unit(const Params& P, int e, int pair, uint16_t* xa, int k0) {

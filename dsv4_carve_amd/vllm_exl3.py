@@ -64,9 +64,9 @@ SWIGLU_LIMIT_DEFAULT = 10.0
 # constant of that name to another value than this module's gets that hand-over
 # for every matrix.  At this module's value it is GEMM_MAX_ROWS, or earlier for
 # wide and expensive matrices.  On MI355X, us per call, decode GEMM /
-# reconstruct: 4096x4096 4-bit 256 rows 34 / 40, 384 rows 48 / 44; 4096x12288
-# 6-bit 256 rows 73 / 89, 512 rows 149 / 106; 1536x4096 256 rows 20 / 29, 512
-# rows 38 / 35; 8192x8192 256 rows 81 / 116, 384 rows 125 / 110.  From
+# reconstruct at 6 bits: 4096x4096 256 rows 30 / 38, 384 rows 49 / 42;
+# 4096x12288 256 rows 75 / 86, 384 rows 117 / 93; 2048x4096 256 rows 21 / 30, 384
+# rows 37 / 31; 8192x8192 256 rows 88 / 118, 384 rows 133 / 118.  From
 # FUSED_RECONSTRUCT_MIN_ROWS rows the rotations are folded into the
 # reconstructed weight (the reference's rule, exl3.py.lna:184).
 AUTO_RECONSTRUCT_THRESHOLD = ops.GEMV_MAX_ROWS
