@@ -106,10 +106,13 @@ int exl3_had_rows(const void* x, int x_kind, void* y, int y_kind, int64_t rows, 
 int64_t exl3_gemm_scratch_bytes(int64_t m, int64_t k, int64_t n) {
     clear_error();
     if (m <= 0 || k <= 0 || n <= 0) return fail("dimensions must be positive");
-    // enough for every call of up to m rows: a k-chunk count may fall as the rows grow
+    // enough for every call of up to m rows: a k-chunk count may fall as the rows
+    // grow (above 32 rows the plan changes with the 16-row blocks only)
     const int cus = device_cus();
-    int64_t most = 0;
-    for (int64_t r = 1; r <= m && r <= GEMM_MAX_ROWS; ++r) most = std::max(most, dense_scratch_bytes(r, k, n, cus));
+    const int64_t last = std::min<int64_t>(m, GEMM_MAX_ROWS);
+    int64_t most = dense_scratch_bytes(last, k, n, cus);
+    for (int64_t r = 1; r < last; r += r < GEMV_MAX_ROWS ? 1 : 16)
+        most = std::max(most, dense_scratch_bytes(r, k, n, cus));
     return most;
 }
 

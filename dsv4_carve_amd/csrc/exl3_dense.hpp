@@ -811,16 +811,20 @@ inline GemmPlan gemm_plan(int64_t R, int64_t k, int64_t n, int cus) {
     // 4096x12288 5-bit 208 rows 82 / 75, where the reconstruct path takes 78); a
     // gain of less than 5% by this model measured between 0.95x and 1.06x, so it is
     // not taken.
+    // Everything here depends on the rows' 16-row blocks only, which
+    // exl3_gemm_scratch_bytes relies on.
+    const int blocks = (int)((R + 15) / 16);
     double best = 1e30;
     for (int n_rt = rt0; n_rt <= rt0 + 1; ++n_rt) {
-        const int rows = (int)((R + n_rt - 1) / n_rt), rb = std::max((rows + 15) / 16, 2);
+        const int rb = std::max((blocks + n_rt - 1) / n_rt, 2);
         const double ts = 0.75 + 0.13 * rb;
         for (int kc = 1; kc <= 32 && kc <= S; ++kc) {
             const int ns = (S + kc - 1) / kc, n_kc = (S + ns - 1) / ns;
             if (n_kc != kc) continue;
             const int64_t wgs = (int64_t)p.n_hb * GEMV_NCG * n_rt * n_kc;
             const double rounds = (double)((wgs + cus - 1) / cus);
-            double t = rounds * (1.5 + ts * ((ns + GEMM_NKG - 1) / GEMM_NKG)) + 2e-6 * n_kc * (double)R * (double)n;
+            double t = rounds * (1.5 + ts * ((ns + GEMM_NKG - 1) / GEMM_NKG)) +
+                       2e-6 * n_kc * (16.0 * blocks) * (double)n;
             if (n_rt > rt0) t /= 0.95;
             if (t < best) {
                 best = t;

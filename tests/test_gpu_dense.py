@@ -452,6 +452,29 @@ def test_many_rows_of_other_types_are_the_cast_ones(ops, dev, k, n, rows):
                 ops.gemm_rows_into(bad, t, u, v, torch.empty((bad.shape[0], n), device=dev))
 
 
+@pytest.mark.parametrize("k,n", [(4096, 256), (1024, 2560), (1280, 8960)])
+def test_scratch_of_a_row_count_serves_every_smaller_one(ops, dev, k, n):
+    """Calls of 1 to 256 rows accept what exl3_gemm_scratch_bytes gives for the
+    same or a larger row count."""
+    import torch
+
+    from dsv4_carve_amd import _lib
+
+    lib = _lib.load()
+    L = synth.dense(k, n, 2, seed=65)
+    t, u, v = (to_dev(L[key], dev) for key in ("trellis", "suh", "svh"))
+    x = to_dev(synth.activations(256, k, seed=66), dev)
+    size = [_lib.check(lib.exl3_gemm_scratch_bytes(m, k, n)) for m in range(1, 301)]
+    assert size == sorted(size)
+    c = torch.empty((256, n), dtype=torch.float32, device=dev)
+    scratch = torch.empty(size[-1], dtype=torch.uint8, device=dev)
+    stream = torch.cuda.current_stream().cuda_stream
+    for m in range(1, 257):
+        _lib.check(lib.exl3_gemm(x.data_ptr(), m, k, t.data_ptr(), n, 2, ops.CB_MCG, u.data_ptr(), v.data_ptr(),
+                                 c.data_ptr(), 2, scratch.data_ptr(), size[m - 1], stream))
+    torch.cuda.synchronize()
+
+
 def test_many_row_linear_reads_its_input_type(dev):
     """A linear of 33-256 bf16 or fp32 rows launches no cast, and gives the
     bits of the cast input's call."""
