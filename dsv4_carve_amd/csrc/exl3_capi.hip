@@ -127,10 +127,13 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
     if (n <= 0 || n % 128) return fail("n must be a positive multiple of 128");
     if (c_kind < OUT_F16 || c_kind > OUT_F32) return fail("c_kind must be 0 (fp16), 1 (bf16) or 2 (fp32)");
     const int cus = device_cus();
-    if (scratch_bytes < dense_scratch_bytes(m, k, n, cus)) return fail("scratch too small");
+    const bool gemm = gemm_takes(m, k, n), one_block = !gemm && m <= GEMV_MAX_ROWS;
+    GemvPlan plan{};
+    if (one_block) plan = gemv_plan(m, k, n, cus);
+    if (scratch_bytes < (one_block ? gemv_scratch_bytes(plan, m) : dense_scratch_bytes(m, k, n, cus)))
+        return fail("scratch too small");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const size_t c_elem = c_kind == OUT_F32 ? 4 : 2;
-    const bool gemm = gemm_takes(m, k, n);
     const int64_t slab = gemm ? GEMM_MAX_ROWS : GEMV_MAX_ROWS;
     for (int64_t r0 = 0; r0 < m; r0 += slab) {
         const int R = (int)std::min(m - r0, slab);
@@ -141,7 +144,7 @@ int exl3_gemm(const uint16_t* a, int64_t m, int64_t k, const int16_t* b, int64_t
             if ((rc = gemm_slab(ar, OUT_F16, R, k, b, n, bits, codebook, suh, svh, cr, c_kind, scratch, cus, s))) return rc;
             continue;
         }
-        const GemvPlan p = gemv_plan(R, k, n, cus);
+        const GemvPlan p = one_block ? plan : gemv_plan(R, k, n, cus);
         float* partials = reinterpret_cast<float*>(scratch);
         const GemvArgs args{ar, b, suh, svh, cr, c_kind, R, (int)k, (int)n, p, codebook, partials, s};
         EXL3_BITS_SWITCH(bits, rc = launch_gemv<B_>(args));

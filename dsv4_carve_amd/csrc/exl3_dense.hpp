@@ -841,11 +841,14 @@ inline GemmPlan gemm_plan(int64_t R, int64_t k, int64_t n, int cus) {
     return p;
 }
 
+inline int64_t gemv_scratch_bytes(const GemvPlan& p, int64_t rows) {
+    return align_up(gemv_partial_bytes(rows, p.n_hb, p.n_kc), 256) + 256;
+}
+
 // Scratch of exactly this call.
 inline int64_t dense_scratch_bytes(int64_t rows, int64_t k, int64_t n, int cus) {
     if (!gemm_takes(rows, k, n)) {
-        const GemvPlan p = gemv_plan(rows, k, n, cus);
-        const int64_t b = align_up(gemv_partial_bytes(rows, p.n_hb, p.n_kc), 256) + 256;
+        const int64_t b = gemv_scratch_bytes(gemv_plan(rows, k, n, cus), rows);
         return rows > GEMV_MAX_ROWS && rows % GEMV_MAX_ROWS
                    ? std::max(b, dense_scratch_bytes(rows % GEMV_MAX_ROWS, k, n, cus))    // the last block
                    : b;

@@ -190,12 +190,13 @@ def _gemm_impl(a, b, c, suh, svh, codebook, scratch):
     m, k = a.shape
     n = b.shape[1] * 16
     bits = b.shape[2] // 16
-    rest = (m, k, _ptr(b), n, bits, int(codebook), _ptr(suh), _ptr(svh), _ptr(c), OUT_KIND[c.dtype], _ptr(scratch),
-            scratch.numel(), _stream(a.device))
-    if a.dtype == torch.float16:
-        _lib.check(L.exl3_gemm(_ptr(a), *rest))
+    if a.dtype is torch.float16:
+        _lib.check(L.exl3_gemm(_ptr(a), m, k, _ptr(b), n, bits, int(codebook), _ptr(suh), _ptr(svh),
+                               _ptr(c), OUT_KIND[c.dtype], _ptr(scratch), scratch.numel(), _stream(a.device)))
     else:
-        _lib.check(L.exl3_gemm_rows(_ptr(a), OUT_KIND[a.dtype], *rest))
+        _lib.check(L.exl3_gemm_rows(_ptr(a), OUT_KIND[a.dtype], m, k, _ptr(b), n, bits, int(codebook), _ptr(suh),
+                                    _ptr(svh), _ptr(c), OUT_KIND[c.dtype], _ptr(scratch), scratch.numel(),
+                                    _stream(a.device)))
 
 
 def _route_args(ids, w, emap):

@@ -112,7 +112,7 @@ def decode_max_rows(k: int, n: int, codebook: int) -> int:
     """Most rows of a [k] -> [n] linear that the decode kernels serve."""
     if AUTO_RECONSTRUCT_THRESHOLD != ops.GEMV_MAX_ROWS:
         return AUTO_RECONSTRUCT_THRESHOLD
-    return gemm_max_rows(k, n, codebook)
+    return max(AUTO_RECONSTRUCT_THRESHOLD, gemm_max_rows(k, n, codebook))
 
 
 class LinearEXL3:
@@ -179,8 +179,9 @@ class LinearEXL3:
         assert x.is_contiguous(), f"LinearEXL3 {self.key}: non-contiguous input {tuple(x.shape)}"
         dtype = out_dtype or self.default_out_dtype
         rows = x.numel() // x.shape[-1]
-        if not params.get("reconstruct") and (self.config.infer_params.no_reconstruct or rows <= decode_max_rows(
-                self.in_features, self.out_features, self.codebook)):
+        if not params.get("reconstruct") and (
+                rows <= AUTO_RECONSTRUCT_THRESHOLD or self.config.infer_params.no_reconstruct
+                or rows <= decode_max_rows(self.in_features, self.out_features, self.codebook)):
             x2 = x.view(rows, self.in_features)
             gemm = ops.gemm_into
             if x2.dtype != torch.float16:
