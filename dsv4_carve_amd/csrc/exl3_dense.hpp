@@ -427,7 +427,7 @@ inline GemvPlan gemv_plan_hb(int64_t rows, int64_t k, int64_t total_hb, int cus)
     // and the steps' decode and rotation.  Only chunks of 8 steps and more: below
     // that the first choice holds four waves a SIMD already.  One round is left as
     // it is unless the gain is clear.  On 63 shapes (512x256 to 4096x129280, 1-32
-    // rows, 1-6 bits) at most 2% slower than the first choice with eight k-groups,
+    // rows, 2-6 bits) at most 2% slower than the first choice with eight k-groups,
     // which one-wave items of whole tiles had beaten by up to 15% there; us, those
     // items / eight k-groups / this rule: 512x129280 2-bit 1 row 14.8 / 17.4 / 12.4;
     // 4096x65536 2-bit 1 row 37.9 / 42.1 / 37.9; 4096x129280 6-bit 1 row 100 / 103 /

@@ -290,8 +290,8 @@ def test_linear_method_prewarms_groups_and_captures(dev):
     module's shards run as one fused call, the scratch is reserved for every
     decode row count (no prepare_gemm by hand), and a graph captured at each
     row count 1..16 replays to the oracle's result; so do graphs at 24 and 32
-    rows, where the group declines and each shard takes the GEMV (which runs
-    up to AUTO_RECONSTRUCT_THRESHOLD rows), with no scratch grown by the
+    rows, where the group declines and each shard takes a dense call on the
+    shared scratch (reserved up to 32 rows), with no scratch grown by the
     capture."""
     import torch
     from dsv4_carve_amd import ops, vllm_exl3 as V

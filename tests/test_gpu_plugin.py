@@ -1,6 +1,6 @@
 """GPU parity of the plugin call surface (dsv4_carve_amd.vllm_exl3) against the
-oracle: LinearEXL3.forward on its three paths (the GEMV up to
-AUTO_RECONSTRUCT_THRESHOLD rows, row Hadamards around an hgemm on Wq up to
+oracle: LinearEXL3.forward on its three paths (the decode kernels up to
+decode_max_rows rows, row Hadamards around an hgemm on Wq up to
 1024 rows, the folded weight beyond), Exl3LinearMethod with several output shards,
 apply_exl3_experts through the routed kernel and through the LinearEXL3 loop,
 expert_map remapping, decline / strict behaviour and the full Exl3MoEMethod
